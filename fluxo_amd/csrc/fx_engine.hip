@@ -630,13 +630,19 @@ int fx_volume_tile(int N, int parabolic, int precision, int *epb)
 int fx_use_volume_tile(fx_ctx *c, int epb)
 {
   if (!c) return set_err(FX_EINVAL, "null context");
-  const int N = c->b.cfg.N, nt = (c->b.cfg.volumeFlux == 32) ? 3 : 1;
-  for (int t = 0; t < nt; t++)
-    if (tile_epb(N, t) == epb) {
-      c->b.vol_tile = t;
-      if (c->graph) { (void)hipGraphExecDestroy(c->graph); c->graph = nullptr; }
-      return FX_OK;
-    }
+  const int N = c->b.cfg.N;
+  const int prec = c->b.cfg.precision, dflt = default_tile(N, prec);
+  const bool ranocha = c->b.cfg.volumeFlux == 32;
+  // the other fluxes run their precision's default; tile 0 is accepted for them too and changes
+  // nothing.  Tile 3 (N = 3) is the FP64 kernel's.
+  for (int t = 0; t < 4; t++) {
+    if (tile_epb(N, t) != epb || epb == 0) continue;
+    if (t == 3 && prec == FX_PREC_FP32_SPLIT) continue;
+    if (!ranocha && t != 0 && t != dflt) continue;
+    if (ranocha) c->b.vol_tile = t;
+    if (c->graph) { (void)hipGraphExecDestroy(c->graph); c->graph = nullptr; }
+    return FX_OK;
+  }
   return set_err(FX_EINVAL, "no volume tile with %d elements per workgroup for N=%d", epb, N);
 }
 
@@ -647,13 +653,18 @@ int fx_tune_volume(fx_ctx *c, int reps, int *best_epb, int *tiles, double *ms, i
   if (reps < 1) return set_err(FX_EINVAL, "reps < 1");
   Batch &b = c->b;
   const int N = b.cfg.N;
-  const int nt = (b.cfg.volumeFlux == 32) ? 3 : 1;  // only the Ranocha LSERK form has alternatives
+  // only the Ranocha LSERK form has alternatives; the others report their single tile
+  const bool ranocha = b.cfg.volumeFlux == 32;
+  const int nt = ranocha ? TUNER_TILES : 1;
+  auto tile = [&](int k) {
+    return ranocha ? tuner_tile(N, b.cfg.precision, k) : default_tile(N, b.cfg.precision);
+  };
   const size_t nv = vol_doubles(b.cfg);
   double *save = nullptr;
   HIPCHK(hipMalloc((void **)&save, 2 * nv * 8));
   auto cleanup = [&]() { (void)hipFree(save); };
   hipEvent_t e0 = nullptr, e1 = nullptr;
-  int best = 0;
+  int best = tile(0);
   double bestms = 1e300;
   hipError_t err = hipSuccess;
 #define TCHK(x) if ((err = (x)) != hipSuccess) goto fail;
@@ -669,7 +680,7 @@ int fx_tune_volume(fx_ctx *c, int reps, int *best_epb, int *tiles, double *ms, i
     RKArgs rk;
     rk.st = b.st; rk.eprob = nullptr; rk.A = b.rkA[0]; rk.b = b.rkb[0]; rk.first = 1;
     rk.alpha = nullptr; rk.Ffv = nullptr;
-    b.vol_tile = t;
+    b.vol_tile = tile(t);
     q_volume(b, VMODE_RK, rk);  // stage 1 form once (warm-up; fills Ut_tmp)
     rk.A = b.rkA[1]; rk.b = b.rkb[1]; rk.first = 0;
     TCHK(hipEventRecord(e0, b.stream));
@@ -679,9 +690,9 @@ int fx_tune_volume(fx_ctx *c, int reps, int *best_epb, int *tiles, double *ms, i
     float f = 0.0f;
     TCHK(hipEventElapsedTime(&f, e0, e1));
     const double avg = (double)f / reps;
-    if (tiles && t < 4) tiles[t] = tile_epb(N, t);
+    if (tiles && t < 4) tiles[t] = tile_epb(N, tile(t));
     if (ms && t < 4) ms[t] = avg;
-    if (avg < bestms) { bestms = avg; best = t; }
+    if (avg < bestms) { bestms = avg; best = tile(t); }
   }
   TCHK(hipMemcpyAsync(b.U, save, nv * 8, hipMemcpyDeviceToDevice, b.stream));
   TCHK(hipMemcpyAsync(b.Uttmp, save + nv, nv * 8, hipMemcpyDeviceToDevice, b.stream));

@@ -29,6 +29,7 @@ struct Ops {
   double D[MAXN + 1][MAXN + 1];     // D(i,l)         (dg.f90:210)
   double w[MAXN + 1];               // LGL weights
   double L0;                        // L_HatMinus0 = L_HatMinus(0) (dg.f90:228-229)
+  double Dsh[MAXN + 1][MAXN + 1];   // Dvolsurf / 2, for fluxes that come doubled (two_point)
   float Ds32[MAXN + 1][MAXN + 1];   // FP32 copies for the split-precision volume integral
   float Dhat32[MAXN + 1][MAXN + 1];
   // NFVSE shock capturing
@@ -47,6 +48,18 @@ template <> struct OpsOf<float> {
   __device__ static __forceinline__ float ds(const Ops &o, int i, int l) { return o.Ds32[i][l]; }
   __device__ static __forceinline__ float dhat(const Ops &o, int i, int l) { return o.Dhat32[i][l]; }
 };
+// Dvolsurf(i,l) as it multiplies the result of two_point, and the scale of the metric vectors that
+// two_point takes
+template <int VF>
+__device__ __forceinline__ double two_point_ds(const Ops &o, int i, int l)
+{
+  return two_point_halved(VF) ? o.Dsh[i][l] : o.Ds[i][l];
+}
+template <int VF>
+__device__ __forceinline__ double two_point_metric(double m)
+{
+  return two_point_halved(VF) ? 0.5 * m : m;
+}
 // One copy per compilation unit (internal linkage): the library is built from several units
 // that each hold kernels, and every unit's copy is filled by ensure_ops (fx_launch.hpp).
 static __constant__ Ops c_ops[MAXN + 1];
@@ -185,15 +198,25 @@ k_face_table(const int *__restrict__ e2s, const int *__restrict__ s2e, int e0, i
 }
 
 // -----------------------------------------------------------------------------------
-// Launch geometry of the volume kernel: EPB elements per block and W = EPB*(N+1)^2
-// threads per direction rounded up to a multiple of 32 (3*W threads in the line phase).  Tiles[0]
-// is the default EPB of each N; the others are the candidates the volume-kernel tuner
-// times (fx_tune_volume) for the LSERK form with the Ranocha flux.
+// Launch geometry of the volume kernel: EPB elements per block.  T holds the tiles (EPB) of each N
+// that the volume-kernel tuner times (fx_tune_volume) for the LSERK form with the Ranocha flux.
+// DEF64 / DEF32 are the defaults' positions: the node form (FP64, N >= 3) and the line form
+// (FP64 at N = 2, FP32-split).  LSERK kernel of the FP64 Ranocha form, line -> node at these
+// defaults: N = 5 (13^3 elements, Euler) 65 -> 39 us, N = 4 (15 x 14 x 13, Navier-Stokes) 54.9 ->
+// 29.2 us, N = 3 8.5 -> 7.1 us (8^3, Euler) and 161 -> 146 us (32^3, Navier-Stokes); at N = 2
+// (24^3, Navier-Stokes) the line form takes 26.3 us, the node form 28.6 us.
+// The node form's default tile: one wavefront per block at N = 3 (its barriers cost nothing), the
+// fewest wavefronts that fill their lanes at N = 4 (2 elements in 250 of 256 threads; 1 and 3: 32 and
+// 37 us against 30), one element at N = 5 (2: 41 us against 39).
 template <int N> struct VolTiles;
-template <> struct VolTiles<2> { static constexpr int n = 3, T[3] = {7, 14, 3}; };
-template <> struct VolTiles<3> { static constexpr int n = 3, T[3] = {4, 2, 8}; };
-template <> struct VolTiles<4> { static constexpr int n = 3, T[3] = {5, 2, 3}; };
-template <> struct VolTiles<5> { static constexpr int n = 3, T[3] = {3, 1, 2}; };
+template <> struct VolTiles<2> { static constexpr int n = 3, T[4] = {7, 14, 3, 0}, DEF64 = 0, DEF32 = 0; };
+template <> struct VolTiles<3> { static constexpr int n = 4, T[4] = {4, 2, 8, 1}, DEF64 = 3, DEF32 = 0; };
+template <> struct VolTiles<4> { static constexpr int n = 3, T[4] = {5, 2, 3, 0}, DEF64 = 1, DEF32 = 0; };
+template <> struct VolTiles<5> { static constexpr int n = 3, T[4] = {3, 1, 2, 0}, DEF64 = 1, DEF32 = 0; };
+// the degrees whose FP64 volume kernel is the node form (k_volume_node)
+__host__ __device__ constexpr bool volume_node_form(int N) { return N >= 3; }
+// Line form: W = EPB*(N+1)^2 threads per direction rounded up to a multiple of 32 (3*W threads in
+// the line phase).
 // TB threads per block: the 3 W of the line phase, plus one wavefront that sits out the line
 // phase where it gives every node of the block its own thread in the node passes (N=3 with
 // 4 elements: 256 nodes on 256 threads instead of two rounds on 192).
@@ -553,6 +576,178 @@ k_volume(double *__restrict__ U, const VR *__restrict__ Mf, const VR *__restrict
 
 #undef SL
 #undef SA
+
+// Node form of the FP64 volume kernel (N >= 3): one thread per node from its state load to its stage
+// update, no line phase.  Same operation and arguments as k_volume (VolInt_SplitForm,
+// VolInt_visc, SurfInt gather, -sJ, Ut or the LSERK stage update).
+//   phase 1  one work item per face point gathers the element's SurfInt terms into LDS; the node's
+//            flux fields and metric vectors into LDS; the node pass's inputs are loaded
+//   phase 2  after a barrier the thread adds Dvolsurf(pos,l) F(pos,l) over the N other nodes of
+//            each of its three lines to five sums in registers, and finishes its node
+// Every pair is evaluated by both of its nodes: twice the flux arithmetic of the line form, against
+// its n x 5 sums per thread (226-232 VGPR at N = 4, 5: one block of 6 wavefronts per CU), its
+// direction sums and three to five of its six barriers.  The kernel holds 118-128 VGPR (4 waves per
+// SIMD) and is bound by its vector instructions at N = 4, 5 and by memory at N = 3 (633 MB in
+// 142-150 us at 32^3 elements, Navier-Stokes: 4.2-4.4 TB/s against 5.1 TB/s of a 1 GiB copy).
+// NodeGeom: EPB elements per block, T threads.  The lines of a direction are rotations of the node
+// index, so unpadded LDS arrays read without bank conflicts.
+template <int N, int EPB_> struct NodeGeom {
+  static constexpr int n3 = (N + 1) * (N + 1) * (N + 1), EPB = EPB_;
+  static constexpr int T = ((EPB * n3 + 63) / 64) * 64;
+};
+template <int N, int VF, bool PARA, int MODE, int EPB_>
+__global__ void __launch_bounds__((NodeGeom<N, EPB_>::T), 4)
+k_volume_node(double *__restrict__ U, const double *__restrict__ Mf, const double *__restrict__ Mg,
+              const double *__restrict__ Mh, const double *__restrict__ sJ, const int *__restrict__ e2s,
+              const double *__restrict__ Flux, const double *__restrict__ Uv, double *__restrict__ Ut,
+              double *__restrict__ Uttmp, RKArgs rk, int nElems, double kappa)
+{
+  constexpr int n = N + 1, n2 = n * n, n3 = n2 * n, NF = 6 * n2;
+  constexpr int EPB = EPB_, T = NodeGeom<N, EPB_>::T, NN = EPB * n3;
+  constexpr int NFV = n_fields<VF>();
+  // FACE1: every node takes its face terms into registers before its fields are staged, so that
+  // the fields reuse their memory.  One more wavefront per SIMD fits at N = 3 (12.6 -> 8.8 KB per
+  // wavefront; LSERK kernel at 40^3 elements, Euler: 263 -> 253 us, 32^3 Navier-Stokes: 156 ->
+  // 146 us) and N = 4 (30.1 -> 29.2 us at 15 x 14 x 13), for two more barriers; at N = 5 the LDS
+  // does not bound the blocks per CU, and the barriers cost 2 us of 39.
+  constexpr bool FACE1 = N <= 4;
+  constexpr int NFACE = MODE != VMODE_VOLINT ? EPB * NF * 5 : 0, NBUF = (NFV + 9) * NN;
+  // node fields [NFV], metric vectors [9, component 3 d + c of direction d] (NN doubles each)
+  __shared__ double s_buf[FACE1 ? (NBUF > NFACE ? NBUF : NFACE) : NBUF + NFACE];
+  __shared__ double s_ds[N][n];  // s_ds[s - 1][pos] = Dvolsurf(pos, (pos + s) mod n)
+  double *s_f = s_buf, *s_m = s_buf + NFV * NN, *s_face = FACE1 ? s_buf : s_buf + NBUF;
+  const Ops &op = c_ops[N];
+  const int tid = threadIdx.x, e0 = blockIdx.x * EPB;
+  const double kappaM1 = kappa - 1.0;
+  const double skappaM1 = 1.0 / kappaM1;
+  const int el = tid / n3, node = tid - el * n3, e = e0 + el;
+  const int prob = (tid < NN && e < nElems) ? elem_problem(rk.eprob, e) : -1;
+  const bool active = prob >= 0;
+  const size_t c = (size_t)e * n3 + node;
+
+  if (tid < N * n) {
+    const int s1 = tid / n, p1 = tid - s1 * n, l1 = p1 + s1 + 1;
+    s_ds[s1][p1] = two_point_ds<VF>(op, p1, l1 < n ? l1 : l1 - n);
+  }
+  const int i = node % n, j = (node / n) % n, k = node / n2;
+  double u[5], m[9], tt[5], uv[4], sj = 0.0;
+  if (active) {
+#pragma unroll
+    for (int v = 0; v < 5; v++) u[v] = U[c * 5 + v];
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+      m[q] = Mf[c * 3 + q];
+      m[3 + q] = Mg[c * 3 + q];
+      m[6 + q] = Mh[c * 3 + q];
+    }
+  }
+  double fs[5] = {0.0, 0.0, 0.0, 0.0, 0.0};  // the node's surface terms
+  auto face_terms = [&]() {
+    const NodeFaces nf = node_faces<N>(i, j, k);
+#pragma unroll
+    for (int t = 0; t < 3; t++) {
+      const int r = nf.get(t);
+      if (r < 0) continue;
+#pragma unroll
+      for (int v = 0; v < 5; v++) fs[v] = fs[v] + s_face[(el * NF + r) * 5 + v];
+    }
+  };
+  if (MODE != VMODE_VOLINT) {
+    // SurfInt terms +-Flux L_HatMinus0 (master +, slave -; surfint.f90:177-184, 253-259) in
+    // element-local face coordinates
+    const double L0 = op.L0;
+#pragma unroll
+    for (int it = tid; it < EPB * NF; it += T) {
+      const int fe = it / NF, r = it - fe * NF, face = r / n2, ab = r - face * n2, ee = e0 + fe;
+      if (ee >= nElems || elem_problem(rk.eprob, ee) < 0) continue;
+      const int loc = face + 1, fnode = face_node<N>(loc, ab % n, ab / n);
+      const int sd = e2s[(ee * 6 + face) * 2] - 1, fl = e2s[(ee * 6 + face) * 2 + 1];
+      int p, q;
+      vol_to_side<N>(loc, fl, fnode % n, (fnode / n) % n, fnode / n2, p, q);
+      const double *F = Flux + ((size_t)(sd * n + q) * n + p) * 5;
+      const double sg = (fl == 0) ? L0 : -L0;
+#pragma unroll
+      for (int v = 0; v < 5; v++) s_face[it * 5 + v] = F[v] * sg;
+    }
+    if (FACE1) {
+      __syncthreads();
+      if (active) face_terms();
+      __syncthreads();
+    }
+  }
+  double own[NF_COUNT];
+  if (active) {
+    node_fields<VF>(u, kappaM1, own);
+#pragma unroll
+    for (int q = 0; q < NF_COUNT; q++)
+      if (uses_field<VF>(q)) s_f[field_slot<VF>(q) * NN + tid] = own[q];
+#pragma unroll
+    for (int q = 0; q < 9; q++) s_m[q * NN + tid] = two_point_metric<VF>(m[q]);
+    if (MODE != VMODE_VOLINT) {
+      sj = sJ[c];
+      if (PARA) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) uv[q] = Uv[c * 4 + q];
+      }
+      if (MODE == VMODE_RK) {
+#pragma unroll
+        for (int v = 0; v < 5; v++) tt[v] = rk.first ? 0.0 : Uttmp[c * 5 + v];
+      }
+    }
+  }
+  __syncthreads();
+  if (!active) return;
+  double tot[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll 1
+  for (int d = 0; d < 3; d++) {
+    const int pos = (d == 0) ? i : ((d == 1) ? j : k), stride = (d == 0) ? 1 : ((d == 1) ? n : n2);
+    const double *sm = s_m + 3 * d * NN;
+    const double mo[3] = {sm[tid], sm[NN + tid], sm[2 * NN + tid]};
+#pragma unroll
+    for (int s = 1; s < n; s++) {
+      const int t2 = tid + (pos + s < n ? s : s - n) * stride;
+      double nb[NF_COUNT], mn[3], F[5];
+#pragma unroll
+      for (int q = 0; q < NF_COUNT; q++) nb[q] = uses_field<VF>(q) ? s_f[field_slot<VF>(q) * NN + t2] : 0.0;
+#pragma unroll
+      for (int q = 0; q < 3; q++) mn[q] = sm[q * NN + t2];
+      two_point<VF>(own, nb, mo, mn, skappaM1, F);
+      const double ds = s_ds[s - 1][pos];
+#pragma unroll
+      for (int v = 0; v < 5; v++) tot[v] += ds * F[v];
+    }
+  }
+  if (rk.alpha) {
+    // VolInt_NFVSE (nfvse.f90:550): Ut = (1 - alpha) Ut + alpha F_FV on the volume part
+    const double a = rk.alpha[e];
+    if (a != 0.0) {
+      const double *ff = rk.Ffv + c * 5;
+#pragma unroll
+      for (int v = 0; v < 5; v++) tot[v] = (1.0 - a) * tot[v] + a * ff[v];
+    }
+  }
+  if (MODE != VMODE_VOLINT) {
+    if (PARA) {  // VolInt_visc, formed by the lifting kernel
+#pragma unroll
+      for (int q = 0; q < 4; q++) tot[q + 1] = tot[q + 1] + uv[q];
+    }
+    if (!FACE1) face_terms();
+#pragma unroll
+    for (int v = 0; v < 5; v++) tot[v] = (tot[v] + fs[v]) * -sj;
+  }
+  if (MODE == VMODE_RK) {
+    const double bdt = rk.b * rk.st[prob].dt;
+#pragma unroll
+    for (int v = 0; v < 5; v++) {
+      const double ut = rk.first ? tot[v] : tt[v] * (-rk.A) + tot[v];
+      Uttmp[c * 5 + v] = ut;
+      U[c * 5 + v] = u[v] + ut * bdt;
+    }
+  } else {
+#pragma unroll
+    for (int v = 0; v < 5; v++) Ut[c * 5 + v] = tot[v];
+  }
+}
 
 // SurfInt alone (surfint.f90:48-264, Gauss-Lobatto branch :177-184, 253-259): Ut +=
 // Flux_master L_HatMinus0 at the master element's face nodes and Ut -= Flux_slave L_HatMinus0

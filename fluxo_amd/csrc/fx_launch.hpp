@@ -153,6 +153,7 @@ inline void make_ops(int N, Ops &o)
   o.L0 = Lm[0] / w[0];
   for (int i = 0; i <= MAXN; i++)
     for (int j = 0; j <= MAXN; j++) {
+      o.Dsh[i][j] = 0.5 * o.Ds[i][j];
       o.Ds32[i][j] = (float)o.Ds[i][j];
       o.Dhat32[i][j] = (float)o.Dhat[i][j];
     }
@@ -331,14 +332,8 @@ inline double dfl_number(int N, double DFLscale)
   return DFLscale * dfl_alpha(N) / ((2.0 * N + 1.0) * (2.0 * N + 1.0));
 }
 
-// Process-wide tile choice (index into VolTiles<N>::T) of the LSERK volume kernel for each
-// degree, Euler/Navier-Stokes and precision: set by the tuner, read when a context or server
-// pool is created.
-inline int &tuned_tile(int N, int parabolic, int precision)
-{
-  static int t[MAXN + 1][2][2] = {};
-  return t[N][parabolic ? 1 : 0][precision == FX_PREC_FP32_SPLIT ? 1 : 0];
-}
+// The tiles of the LSERK volume kernel (VolTiles<N>): elements per block of tile idx (0: none), the
+// tuner's candidates and the default's index for a precision.
 inline int tile_epb(int N, int idx)
 {
   switch (N) {
@@ -348,6 +343,42 @@ inline int tile_epb(int N, int idx)
   case 5: return VolTiles<5>::T[idx];
   default: return 0;
   }
+}
+// The tuner's k-th candidate (k < TUNER_TILES): the default and two others.
+constexpr int TUNER_TILES = 3;
+inline int tuner_tile(int N, int precision, int k)
+{
+  return (N == 3 && precision != FX_PREC_FP32_SPLIT) ? (VolTiles<3>::DEF64 + k) % VolTiles<3>::n : k;
+}
+inline int default_tile(int N, int precision)
+{
+  const bool f32 = precision == FX_PREC_FP32_SPLIT;
+  switch (N) {
+  case 2: return f32 ? VolTiles<2>::DEF32 : VolTiles<2>::DEF64;
+  case 3: return f32 ? VolTiles<3>::DEF32 : VolTiles<3>::DEF64;
+  case 4: return f32 ? VolTiles<4>::DEF32 : VolTiles<4>::DEF64;
+  case 5: return f32 ? VolTiles<5>::DEF32 : VolTiles<5>::DEF64;
+  default: return 0;
+  }
+}
+// Process-wide tile choice (index into VolTiles<N>::T) of the LSERK volume kernel for each
+// degree, Euler/Navier-Stokes and precision: set by the tuner, read when a context or server
+// pool is created.
+inline int &tuned_tile(int N, int parabolic, int precision)
+{
+  struct Choice {
+    int t[MAXN + 1][2][2];
+    Choice()
+    {
+      for (int n = 0; n <= MAXN; n++)
+        for (int p = 0; p < 2; p++) {
+          t[n][p][0] = default_tile(n, FX_PREC_FP64);
+          t[n][p][1] = default_tile(n, FX_PREC_FP32_SPLIT);
+        }
+    }
+  };
+  static Choice c;
+  return c.t[N][parabolic ? 1 : 0][precision == FX_PREC_FP32_SPLIT ? 1 : 0];
 }
 
 // blocks of a lifting launch (LiftGeom<N>::EPB elements each)

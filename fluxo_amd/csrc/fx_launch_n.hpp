@@ -9,33 +9,42 @@ namespace fx {
 template <int N, int VF, bool PARA, int MODE, int EPB>
 void launch_volume_e(const Batch &b, RKArgs rk)
 {
-  using G = VolGeom<N, EPB>;
   const int nb = (b.cfg.nElems + EPB - 1) / EPB;
   if (nb <= 0) return;
   if constexpr (has_fp32(VF)) {
     if (b.cfg.precision == FX_PREC_FP32_SPLIT) {
-      hipLaunchKernelGGL((k_volume<N, VF, PARA, MODE, float, EPB>), dim3(nb), dim3(G::TB), 0, b.stream, b.U,
-                         b.Mf32, b.Mg32, b.Mh32, b.sJ, b.e2s, b.Flux, b.Uv, b.Ut, b.Uttmp, rk, b.cfg.nElems,
+      hipLaunchKernelGGL((k_volume<N, VF, PARA, MODE, float, EPB>), dim3(nb), dim3(VolGeom<N, EPB>::TB), 0, b.stream,
+                         b.U, b.Mf32, b.Mg32, b.Mh32, b.sJ, b.e2s, b.Flux, b.Uv, b.Ut, b.Uttmp, rk, b.cfg.nElems,
                          b.cfg.kappa);
       return;
     }
   }
-  hipLaunchKernelGGL((k_volume<N, VF, PARA, MODE, double, EPB>), dim3(nb), dim3(G::TB), 0, b.stream, b.U,
-                       b.Mf, b.Mg, b.Mh, b.sJ, b.e2s, b.Flux, b.Uv, b.Ut, b.Uttmp, rk, b.cfg.nElems,
+  if constexpr (volume_node_form(N))
+    hipLaunchKernelGGL((k_volume_node<N, VF, PARA, MODE, EPB>), dim3(nb), dim3(NodeGeom<N, EPB>::T), 0, b.stream, b.U,
+                       b.Mf, b.Mg, b.Mh, b.sJ, b.e2s, b.Flux, b.Uv, b.Ut, b.Uttmp, rk, b.cfg.nElems, b.cfg.kappa);
+  else
+    hipLaunchKernelGGL((k_volume<N, VF, PARA, MODE, double, EPB>), dim3(nb), dim3(VolGeom<N, EPB>::TB), 0, b.stream,
+                       b.U, b.Mf, b.Mg, b.Mh, b.sJ, b.e2s, b.Flux, b.Uv, b.Ut, b.Uttmp, rk, b.cfg.nElems,
                        b.cfg.kappa);
 }
 
-// The LSERK form with the Ranocha flux has every tile of VolTiles<N>; other forms use the
-// default tile.
+// The LSERK form with the Ranocha flux has every tile of VolTiles<N>; other forms use their
+// precision's default tile.
 template <int N, int VF, bool PARA, int MODE>
 void launch_volume_t(const Batch &b, RKArgs rk)
 {
-  constexpr int T0 = VolTiles<N>::T[0], T1 = VolTiles<N>::T[1], T2 = VolTiles<N>::T[2];
-  if (MODE == VMODE_RK && VF == 32) {
-    if (b.vol_tile == 1) { launch_volume_e<N, VF, PARA, MODE, T1>(b, rk); return; }
-    if (b.vol_tile == 2) { launch_volume_e<N, VF, PARA, MODE, T2>(b, rk); return; }
+  using V = VolTiles<N>;
+  if constexpr (MODE == VMODE_RK && VF == 32) {
+    switch (b.vol_tile) {
+    case 1: launch_volume_e<N, VF, PARA, MODE, V::T[1]>(b, rk); break;
+    case 2: launch_volume_e<N, VF, PARA, MODE, V::T[2]>(b, rk); break;
+    case 3: launch_volume_e<N, VF, PARA, MODE, V::T[V::n - 1]>(b, rk); break;  // tile 3 exists where n = 4
+    default: launch_volume_e<N, VF, PARA, MODE, V::T[0]>(b, rk); break;
+    }
+    return;
   }
-  launch_volume_e<N, VF, PARA, MODE, T0>(b, rk);
+  if (b.cfg.precision == FX_PREC_FP32_SPLIT) launch_volume_e<N, VF, PARA, MODE, V::T[V::DEF32]>(b, rk);
+  else launch_volume_e<N, VF, PARA, MODE, V::T[V::DEF64]>(b, rk);
 }
 
 template <int N, int VF>

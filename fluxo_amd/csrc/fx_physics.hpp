@@ -17,7 +17,7 @@
 
 namespace fx {
 
-constexpr double LNMEAN_EPS = 1.0e-4;
+constexpr double LNMEAN_SQEPS = 1.0e-2;  // the reference's switch u = ((b-a)/(a+b))^2 < 1e-4
 
 // Reciprocal from the hardware estimate refined by one Newton step (error ~1 ulp); used
 // where a correctly rounded quotient is not needed for FP64 parity at 1e-12.
@@ -29,36 +29,33 @@ __device__ __forceinline__ double rcp_nr(double x)
 }
 __device__ __forceinline__ float rcp_nr(float x) { return __builtin_amdgcn_rcpf(x); }
 
-// Log mean of a, b given la = ln a, lb = ln b, evaluated without branches: both the
-// near-equal series and the log quotient are formed and one is selected, so divergent
-// lanes cost one quotient instead of both paths.  u = ((b-a)/(b+a))^2 only feeds the
-// series (u < 1e-4 there), where its ~1-ulp reciprocal error is below 1e-20.
-template <typename R>
-__device__ __forceinline__ void ln_mean_parts(R a, R b, R la, R lb, R &num, R &den)
-{
-  const R d = b - a, s = a + b, d2 = d * d, s2 = s * s;
-  const R u = d2 * rcp_nr(s2);
-  const R P = R(105.0) + u * (R(35.0) + u * (R(21.0) + u * R(15.0)));
-  const bool series = d2 < R(LNMEAN_EPS) * s2;
-  num = series ? s * R(52.5) : d;
-  den = series ? P : (lb - la);
-}
-
+// Log mean of a, b given la = ln a, lb = ln b, evaluated without branches: the near-equal series
+// and the log quotient are formed and one is selected, so divergent lanes cost one quotient instead
+// of both paths.  Both share one reciprocal (of a + b for the series, of the quotient's
+// denominator otherwise): with q = (b-a)/(a+b) and u = q^2 < 1e-4 the reference's series
+// 52.5 (a+b) / (105 + 35 u + 21 u^2 + 15 u^3) is (a+b) times its own expansion in u, whose
+// neglected u^4 term is below 4e-18.
 template <typename R>
 __device__ __forceinline__ R ln_mean(R a, R b, R la, R lb)
 {
-  R num, den;
-  ln_mean_parts(a, b, la, lb, num, den);
-  return num * rcp_nr(den);
+  const R d = b - a, s = a + b;
+  const bool series = fabs(d) < fabs(R(LNMEAN_SQEPS) * s);
+  const R q = d * rcp_nr(series ? s : lb - la);
+  const R u = q * q;
+  const R P = R(0.5) - u * (R(1.0 / 6.0) + u * (R(2.0 / 45.0) + u * R(22.0 / 945.0)));
+  return series ? s * P : q;
 }
 
 // 1 / ln_mean(a, b)
 template <typename R>
 __device__ __forceinline__ R inv_ln_mean(R a, R b, R la, R lb)
 {
-  R num, den;
-  ln_mean_parts(a, b, la, lb, num, den);
-  return den * rcp_nr(num);
+  const R d = b - a, s = a + b;
+  const bool series = fabs(d) < fabs(R(LNMEAN_SQEPS) * s);
+  const R r = rcp_nr(series ? s : d);
+  const R q = d * r, u = q * q;
+  const R P = R(2.0) + u * (R(2.0 / 3.0) + u * (R(2.0 / 5.0) + u * R(2.0 / 7.0)));
+  return r * (series ? P : lb - la);
 }
 
 // FP32 log mean of the split-precision volume integral.  The near-equal branch is kept in
@@ -320,6 +317,35 @@ __device__ __forceinline__ void volume_flux(const R *L, const R *Rt, const R *mL
     F[2] = R(0.5) * (L[NF_RHO] * L[NF_V2] * qL + Rt[NF_RHO] * Rt[NF_V2] * qR + mL[1] * L[NF_P] + mR[1] * Rt[NF_P]);
     F[3] = R(0.5) * (L[NF_RHO] * L[NF_V3] * qL + Rt[NF_RHO] * Rt[NF_V3] * qR + mL[2] * L[NF_P] + mR[2] * Rt[NF_P]);
     F[4] = R(0.5) * ((L[NF_E] + L[NF_P]) * qL + (Rt[NF_E] + Rt[NF_P]) * qR);
+  }
+}
+
+// The two-point fluxes as the node-form volume kernel evaluates them.  For the Ranocha flux the
+// factors 1/2 of its means are taken out of the pair loop, which that kernel's vector
+// instructions bound: the metrics come halved (hL, hR, so that {{m}} = hL + hR), the result is twice
+// the flux and belongs with halved operator entries (two_point_ds).  With the means' single
+// reciprocal it takes 64 instead of 87 FP64 instructions (LSERK kernel at N = 5, 13^3 elements: 45 -> 39 us).
+// The other fluxes are volume_flux as it stands.
+__host__ __device__ constexpr bool two_point_halved(int VF) { return VF == 32; }
+template <int VF>
+__device__ __forceinline__ void two_point(const double *L, const double *Rt, const double *hL, const double *hR,
+                                          double skappaM1, double *F)
+{
+  if constexpr (two_point_halved(VF)) {
+    const double m0 = hL[0] + hR[0], m1 = hL[1] + hR[1], m2 = hL[2] + hR[2];
+    const double vmL = L[NF_V1] * m0 + L[NF_V2] * m1 + L[NF_V3] * m2;
+    const double vmR = Rt[NF_V1] * m0 + Rt[NF_V2] * m1 + Rt[NF_V3] * m2;
+    const double ps = L[NF_P] + Rt[NF_P];
+    const double vv = L[NF_V1] * Rt[NF_V1] + L[NF_V2] * Rt[NF_V2] + L[NF_V3] * Rt[NF_V3];
+    const double sx = inv_ln_mean(L[NF_X], Rt[NF_X], L[NF_LNX], Rt[NF_LNX]);
+    const double f0 = ln_mean(L[NF_RHO], Rt[NF_RHO], L[NF_LNRHO], Rt[NF_LNRHO]) * (vmL + vmR), fh = 0.5 * f0;
+    F[0] = f0;
+    F[1] = fh * (L[NF_V1] + Rt[NF_V1]) + m0 * ps;
+    F[2] = fh * (L[NF_V2] + Rt[NF_V2]) + m1 * ps;
+    F[3] = fh * (L[NF_V3] + Rt[NF_V3]) + m2 * ps;
+    F[4] = fh * (vv + sx * (2.0 * skappaM1)) + (L[NF_P] * vmR + Rt[NF_P] * vmL);
+  } else {
+    volume_flux<VF, double>(L, Rt, hL, hR, skappaM1, F);
   }
 }
 
