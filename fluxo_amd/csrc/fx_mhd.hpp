@@ -335,369 +335,124 @@ k_mhd_surface(const double *__restrict__ U, const double *__restrict__ FvN, cons
   for (int v = 0; v < MV; v++) { om[v] = Fm[v] * g.w; os[v] = Fs[v] * g.w; }
 }
 
-// Element-centric GLM-MHD volume kernel (same phases as k_volume).
-// Launch geometry of the GLM-MHD volume kernel: EPB elements per block, one thread per
-// (element, direction, node), T threads rounded up to whole wavefronts.
+// Twice the Derigs flux of a pair, as the volume kernel evaluates it (with halved operator
+// entries): hL, hR are the halved metric vectors, so that {{m}} = hL + hR.  Written in the
+// products of the two states instead of the means: with vmL = v_L.{{m}} and BmL = B_L.{{m}},
+//   2 F4 = 2 F0 (1/(2 (kappa-1) betaLN) + v_L.v_R / 2) + pTilde (vmL + vmR) + smu0/2 [ (vmL + vmR) B_L.B_R +
+//          1/2 (vmL - vmR)(|B_R|^2 - |B_L|^2) - (BmL + BmR)(v_L.B_R + v_R.B_L) + 2 ch (psi_L BmR + psi_R BmL) ],
+// which is derigs_flux with the scalar products of its means multiplied out (their |v|^2 and v.B
+// terms cancel).  BmR, the Powell term's B_R.{{m}}, comes back for the caller.
+template <typename R>
+__device__ __forceinline__ void derigs_flux2(const R *L, const R *Rt, const R *hL, const R *hR, R ch, R smu0, R skm1,
+                                             R *F, R &BmR)
+{
+  const R m0 = hL[0] + hR[0], m1 = hL[1] + hR[1], m2 = hL[2] + hR[2];
+  const R vmL = L[MF_V1] * m0 + L[MF_V2] * m1 + L[MF_V3] * m2;
+  const R vmR = Rt[MF_V1] * m0 + Rt[MF_V2] * m1 + Rt[MF_V3] * m2;
+  const R BmL = L[MF_B1] * m0 + L[MF_B2] * m1 + L[MF_B3] * m2;
+  BmR = Rt[MF_B1] * m0 + Rt[MF_B2] * m1 + Rt[MF_B3] * m2;
+  const R vm = vmL + vmR, Bm = BmL + BmR;
+  const R sv0 = L[MF_V1] + Rt[MF_V1], sv1 = L[MF_V2] + Rt[MF_V2], sv2 = L[MF_V3] + Rt[MF_V3];
+  const R sB0 = L[MF_B1] + Rt[MF_B1], sB1 = L[MF_B2] + Rt[MF_B2], sB2 = L[MF_B3] + Rt[MF_B3];
+  const R hs = R(0.5) * smu0;
+  const R pt = (L[MF_RHO] + Rt[MF_RHO]) * rcp_nr(L[MF_BETA] + Rt[MF_BETA]) + hs * (L[MF_BB] + Rt[MF_BB]);
+  F[0] = ln_mean(L[MF_RHO], Rt[MF_RHO], L[MF_LNRHO], Rt[MF_LNRHO]) * vm;
+  const R fh = R(0.5) * F[0], vh = R(0.5) * vm, Bh = R(0.5) * Bm, bs = smu0 * Bh;
+  F[1] = fh * sv0 - bs * sB0 + pt * m0;
+  F[2] = fh * sv1 - bs * sB1 + pt * m1;
+  F[3] = fh * sv2 - bs * sB2 + pt * m2;
+  const R cp = ch * (L[MF_PSI] + Rt[MF_PSI]);
+  F[5] = vh * sB0 - Bh * sv0 + cp * m0;
+  F[6] = vh * sB1 - Bh * sv1 + cp * m1;
+  F[7] = vh * sB2 - Bh * sv2 + cp * m2;
+  F[8] = ch * Bm;
+  const R sb = inv_ln_mean(L[MF_BETA], Rt[MF_BETA], L[MF_LNBETA], Rt[MF_LNBETA]);
+  const R vv = L[MF_V1] * Rt[MF_V1] + L[MF_V2] * Rt[MF_V2] + L[MF_V3] * Rt[MF_V3];
+  const R BB = L[MF_B1] * Rt[MF_B1] + L[MF_B2] * Rt[MF_B2] + L[MF_B3] * Rt[MF_B3];
+  const R vB = L[MF_V1] * Rt[MF_B1] + L[MF_V2] * Rt[MF_B2] + L[MF_V3] * Rt[MF_B3] + Rt[MF_V1] * L[MF_B1] +
+               Rt[MF_V2] * L[MF_B2] + Rt[MF_V3] * L[MF_B3];
+  const R pB = L[MF_PSI] * BmR + Rt[MF_PSI] * BmL;
+  F[4] = fh * (skm1 * sb + vv) + pt * vh +
+         hs * (vm * BB + (R(0.5) * (vmL - vmR)) * (Rt[MF_BB] - L[MF_BB]) - Bm * vB + (R(2) * ch) * pB);
+}
+
+// Element-centric GLM-MHD volume kernel (VolInt_SplitForm with EvalAdvFluxAverage3D and
+// AddNonConsFluxTilde3D, mhd/flux_average.f90:112-186, 268-366; VolInt_visc; SurfInt; -sJ; the
+// LSERK stage update), FP64 and FP32-split, one thread per node as k_volume_node: face terms into
+// registers, node fields and metric vectors into their LDS, then Dvolsurf(pos,l) F(pos,l) and the
+// Powell term's Dvolsurf(pos,l) B_l.{{m}} over the other nodes of the thread's three lines.
+// Every pair is evaluated by both of its nodes.  Against one thread per (direction, node) that
+// evaluated each pair once and handed the partner its half through LDS (two barriers per pair
+// slot, three direction sums, 63 KB of LDS) and, in FP32, one thread per line (248 VGPR), resistive,
+// per LSERK launch: N = 4 24^3 FP64 377 -> 218 us, 15^3 FP32 71 -> 51 us; N = 2 30^3 151 -> 95 us
+// (FP32 131 -> 89), N = 3 24^3 188 -> 113 us (172 -> 104), N = 5 14^3 172 -> 89 us (105 -> 71).
+// It is bound by memory: 882 MB (24^3, N = 4) at 4.0 TB/s, 5.1 TB/s being the rate of a 1 GiB copy;
+// its vector instructions take about 110 us.  The stage update's stores are issued together,
+// Ut_tmp's and then U's, because interleaved with its loads they left L2 in parts (376 instead of
+// 250 MB written, 294 us), and U's old values come from LDS and the fields instead of memory.
+// Blocks of one element (7 at N = 2); N = 4 with two: 222 us.
 template <int N> struct MhdGeom;
-template <> struct MhdGeom<2> { static constexpr int EPB = 3; };
-template <> struct MhdGeom<3> { static constexpr int EPB = 2; };
+template <> struct MhdGeom<2> { static constexpr int EPB = 7; };
+template <> struct MhdGeom<3> { static constexpr int EPB = 1; };
 template <> struct MhdGeom<4> { static constexpr int EPB = 1; };
 template <> struct MhdGeom<5> { static constexpr int EPB = 1; };
 template <int N> struct MhdVolGeom {
   static constexpr int n3 = (N + 1) * (N + 1) * (N + 1), EPB = MhdGeom<N>::EPB;
-  static constexpr int T = ((EPB * 3 * n3 + 63) / 64) * 64;
+  static constexpr int T = ((EPB * n3 + 63) / 64) * 64;
 };
+// the node fields that derigs_flux2 reads, in LDS slots
+constexpr int MFS_COUNT = 12;
+__host__ __device__ constexpr int mfs_slot(int f) { return f <= MF_LNBETA ? f : MF_LNBETA + 1; }  // MF_BB last
 
-// Element-centric GLM-MHD volume kernel (VolInt_SplitForm with EvalAdvFluxAverage3D and
-// AddNonConsFluxTilde3D, mhd/flux_average.f90:112-186, 268-366; VolInt_visc; SurfInt; -sJ; the
-// LSERK stage update).  One thread per (element, direction d, node k at position pos of its
-// line in direction d).  Each pair of a line is evaluated once, by one of its two nodes: in
-// slot s = 1..n/2 node pos takes the pair (pos, pos + s mod n) (for even n the last slot only
-// for pos < n/2), so every node evaluates at most n/2 two-point Derigs fluxes, the lower line
-// index always the left state.  The thread adds Dvolsurf(pos,l) F and its Powell term to its
-// own sums and leaves Dvolsurf(l,pos) F and the partner's Powell term in an LDS exchange
-// buffer, from which the partner adds them after a barrier (a thread keeps one node's sums).
-//   phase 1  one thread per (element, direction, node): the node fields (direction 0) and the
-//            node's metric of its direction into LDS
-//   phase 2  the flux differencing as above, sums into LDS over the fields (after a barrier)
-//   phase 3  face gather +FluxM L0 / -FluxS L0 into LDS (the memory of the exchange buffer),
-//            then one thread per node: direction sums, viscous volume term, surface terms,
-//            -sJ, Ut or the RK stage update
 template <int N, int MODE, typename VR, bool PARA>
-__global__ void __launch_bounds__(MhdVolGeom<N>::T)
+__global__ void __launch_bounds__(MhdVolGeom<N>::T, sizeof(VR) == 4 ? 4 : 3)
 k_mhd_volume(double *__restrict__ U, const VR *__restrict__ Mf, const VR *__restrict__ Mg, const VR *__restrict__ Mh,
              const double *__restrict__ sJ, const int *__restrict__ e2s, const double *__restrict__ FluxM,
              const double *__restrict__ FluxS, const double *__restrict__ Uv, double *__restrict__ Ut,
              double *__restrict__ Uttmp, RKArgs rk, int nElems, MhdArgs a, const DtState *__restrict__ st)
 {
-  constexpr int n = N + 1, n2 = n * n, n3 = n2 * n;
-  constexpr int EPB = MhdVolGeom<N>::EPB, T = MhdVolGeom<N>::T, NP = Lds<N>::NP;
-  // per element: the node fields and the three metric vectors (phases 1-2), later the three
-  // direction sums (MV values per node each)
-  constexpr int FSLOTS = MF_COUNT + 9, ASLOTS = 3 * MV, SLOTS = FSLOTS > ASLOTS ? FSLOTS : ASLOTS;
-  __shared__ VR s_buf[EPB][SLOTS * NP];
-#define MF_AT(el_, c_, l_) s_buf[el_][(c_) * NP + (l_)]
-#define MM_AT(el_, d_, c_, l_) s_buf[el_][(MF_COUNT + 3 * (d_) + (c_)) * NP + (l_)]
-#define MA_AT(el_, d_, v_, l_) s_buf[el_][(MV * (d_) + (v_)) * NP + (l_)]
+  constexpr int n = N + 1, n2 = n * n, n3 = n2 * n, NF = 6 * n2;
+  constexpr int EPB = MhdVolGeom<N>::EPB, T = MhdVolGeom<N>::T, NN = EPB * n3;
+  // the face terms' memory becomes the node fields' and the metric vectors'
+  constexpr size_t FACEB = MODE != VMODE_VOLINT ? (size_t)EPB * NF * MV * 8 : 0, BUFB = (size_t)(MFS_COUNT + 9) * NN * sizeof(VR);
+  __shared__ __align__(16) unsigned char s_raw[FACEB > BUFB ? FACEB : BUFB];
+  __shared__ VR s_ds[N][n];  // s_ds[s - 1][pos] = Dvolsurf(pos, (pos + s) mod n) / 2
+  // the state's values that the node fields do not hold, for the stage update
+  __shared__ double s_u[MODE == VMODE_RK ? (sizeof(VR) == 8 ? 4 : MV) * NN : 1];
+  VR *s_f = reinterpret_cast<VR *>(s_raw), *s_m = s_f + MFS_COUNT * NN;
+  double *s_face = reinterpret_cast<double *>(s_raw);
   const Ops &op = c_ops[N];
   const int tid = threadIdx.x, e0 = blockIdx.x * EPB;
-  const VR ch = VR(st->glm_ch), smu0 = VR(a.smu0), skm1 = VR(1.0 / (a.kappa - 1.0));
-
-  const int el = tid / (3 * n3), rr = tid - el * (3 * n3), dir = rr / n3, node = rr - dir * n3;
-  const int e = e0 + el;
-  const bool active = (el < EPB) && (e < nElems) && elem_problem(rk.eprob, e) >= 0;
+  const int el = tid / n3, node = tid - el * n3, e = e0 + el;
+  const int prob = (tid < NN && e < nElems) ? elem_problem(rk.eprob, e) : -1;
+  const bool active = prob >= 0;
+  const size_t c = (size_t)e * n3 + node;
   const int i = node % n, j = (node / n) % n, k = node / n2;
-  const int ln = Lds<N>::li(node);
-  // the face gather's fluxes (phase 3), loaded before phase 1 and kept in registers through the
-  // pair slots, whose exchange buffer the face terms later reuse
-#ifndef FX_MHDVOL_GPRE
-#define FX_MHDVOL_GPRE 1
-#endif
-  constexpr int NFP = 6 * n2;
-  constexpr bool GPRE = FX_MHDVOL_GPRE && MODE != VMODE_VOLINT && (EPB * NFP <= T);
-  double gpre[MV];
-  double gsg = 0.0;
-  if (GPRE && tid < EPB * NFP) {
-    const int fe = tid / NFP, r = tid - fe * NFP, face = r / n2, ab = r - face * n2;
-    const int ee = e0 + fe;
-    if (ee < nElems && elem_problem(rk.eprob, ee) >= 0) {
-      const int loc = face + 1, fnode = face_node<N>(loc, ab % n, ab / n);
-      const int sd = e2s[(ee * 6 + face) * 2] - 1, fl = e2s[(ee * 6 + face) * 2 + 1];
-      int p, q;
-      vol_to_side<N>(loc, fl, fnode % n, (fnode / n) % n, fnode / n2, p, q);
-      const size_t f = ((size_t)(sd * n + q) * n + p) * MV;
-      const double *F = (fl == 0) ? FluxM + f : FluxS + f;
-      gsg = (fl == 0) ? op.L0 : -op.L0;
-#pragma unroll
-      for (int v = 0; v < MV; v++) gpre[v] = F[v];
-    }
+  if (tid < N * n) {
+    const int s1 = tid / n, p1 = tid - s1 * n, l1 = p1 + s1 + 1;
+    s_ds[s1][p1] = VR(op.Dsh[p1][l1 < n ? l1 : l1 - n]);
   }
-  if (active) {
-    if (dir == 0) {
-      const double *u = U + ((size_t)e * n3 + node) * MV;
-      double uu[MV], f[MF_COUNT];
-#pragma unroll
-      for (int v = 0; v < MV; v++) uu[v] = u[v];
-      mhd_node_fields(uu, a, f);
-#pragma unroll
-      for (int c = 0; c < MF_COUNT; c++) MF_AT(el, c, ln) = VR(f[c]);
-    }
-    const VR *M = (dir == 0) ? Mf : ((dir == 1) ? Mg : Mh);
-    const VR *mp = M + ((size_t)e * n3 + node) * 3;
-#pragma unroll
-    for (int c = 0; c < 3; c++) MM_AT(el, dir, c, ln) = mp[c];
-  }
-  __syncthreads();
-
-  // exchange buffer of phase 2 (MV flux values and the Powell term per thread), later the
-  // face terms of phase 3
-  constexpr int NF = 6 * n2, NX = (MV + 1) * T, NFACE = MODE != VMODE_VOLINT ? EPB * NF * MV : 1;
-  __shared__ double s_xf[NX > NFACE ? NX : NFACE];
-  VR acc[MV];
-#pragma unroll
-  for (int v = 0; v < MV; v++) acc[v] = VR(0);
-  VR snc = VR(0);
-  const int pos = (dir == 0) ? i : ((dir == 1) ? j : k);  // the node's index along its line
-  const int stride = (dir == 0) ? 1 : ((dir == 1) ? (n + 1) : (n + 1) * n);  // LDS step along the line
-  const int l0 = ln - pos * stride;                        // LDS index of the line's node 0
-  const int tstep = (dir == 0) ? 1 : ((dir == 1) ? n : n2);  // thread step along the line
-  VR fk[MF_COUNT], mk[3];
+  double u[MV];
+  VR m[9];
   if (active) {
 #pragma unroll
-    for (int c = 0; c < MF_COUNT; c++) fk[c] = MF_AT(el, c, ln);
+    for (int v = 0; v < MV; v++) u[v] = U[c * MV + v];
 #pragma unroll
-    for (int c = 0; c < 3; c++) mk[c] = MM_AT(el, dir, c, ln);
-  }
-  constexpr int SLOT_UNROLL = n / 2 <= 2 ? n / 2 : 1;  // N=5 unrolled spills
-#pragma unroll SLOT_UNROLL
-  for (int sl = 1; sl <= n / 2; sl++) {
-    const bool half = (n % 2 == 0) && (sl == n / 2);  // the pairs (p, p + n/2): once each
-    if (active && (!half || pos < n / 2)) {
-      const int l = pos + sl < n ? pos + sl : pos + sl - n;
-      const int ll = l0 + l * stride;
-      VR fl[MF_COUNT], ml[3], F[MV];
-#pragma unroll
-      for (int c = 0; c < MF_COUNT; c++) fl[c] = MF_AT(el, c, ll);
-#pragma unroll
-      for (int c = 0; c < 3; c++) ml[c] = MM_AT(el, dir, c, ll);
-      if (pos < l) derigs_flux<VR>(fk, fl, mk, ml, ch, smu0, skm1, F);
-      else derigs_flux<VR>(fl, fk, ml, mk, ch, smu0, skm1, F);
-      const VR mb0 = VR(0.5) * (mk[0] + ml[0]), mb1 = VR(0.5) * (mk[1] + ml[1]), mb2 = VR(0.5) * (mk[2] + ml[2]);
-      const VR dkl = OpsOf<VR>::ds(op, pos, l), dlk = OpsOf<VR>::ds(op, l, pos);
-#pragma unroll
-      for (int v = 0; v < MV; v++) {
-        acc[v] += dkl * F[v];
-        s_xf[v * T + tid] = dlk * F[v];
-      }
-      // Powell: B_l.{{m}} towards node pos, B_pos.{{m}} towards node l
-      snc += dkl * (mb0 * fl[MF_B1] + mb1 * fl[MF_B2] + mb2 * fl[MF_B3]);
-      s_xf[MV * T + tid] = dlk * (mb0 * fk[MF_B1] + mb1 * fk[MF_B2] + mb2 * fk[MF_B3]);
-    }
-    __syncthreads();
-    if (active && (!half || pos >= n / 2)) {  // the pair (m, pos) taken by node m in this slot
-      const int m = pos - sl >= 0 ? pos - sl : pos - sl + n;
-      const int ts = tid + (m - pos) * tstep;
-#pragma unroll
-      for (int v = 0; v < MV; v++) acc[v] += s_xf[v * T + ts];
-      snc += s_xf[MV * T + ts];
-    }
-    __syncthreads();  // the next slot overwrites the exchange buffer
-  }
-  if (active) {
-    const VR b1 = fk[MF_B1], b2 = fk[MF_B2], b3 = fk[MF_B3];
-    const VR bhat = mk[0] * b1 + mk[1] * b2 + mk[2] * b3;
-    const VR t = VR(0.5) * (bhat * VR(op.DsRow[pos]) + snc);
-    acc[1] += t * b1; acc[2] += t * b2; acc[3] += t * b3;
-    acc[4] += t * fk[MF_VB];
-    acc[5] += t * fk[MF_V1];
-    acc[6] += t * fk[MF_V2];
-    acc[7] += t * fk[MF_V3];
-  }
-  __syncthreads();  // the sums overwrite the fields: every thread must have read them
-  if (active) {
-#pragma unroll
-    for (int v = 0; v < MV; v++) MA_AT(el, dir, v, ln) = acc[v];
-  }
-
-  // the element's SurfInt terms +FluxM L0 (master) / -FluxS L0 (slave) into LDS in
-  // element-local face coordinates, one work item per face point (the exchange buffer is no
-  // longer read: the last slot ended with a barrier)
-  const double L0 = op.L0;
-  auto s_face = reinterpret_cast<double (*)[NF * MV]>(s_xf);
-  if (GPRE) {
-    if (tid < EPB * NF && gsg != 0.0) {
-      const int fe = tid / NF, r = tid - fe * NF;
-#pragma unroll
-      for (int v = 0; v < MV; v++) s_face[fe][r * MV + v] = gpre[v] * gsg;
-    }
-  } else if (MODE != VMODE_VOLINT) {
-    for (int it = tid; it < EPB * NF; it += T) {
-      const int fe = it / NF, r = it - fe * NF, face = r / n2, ab = r - face * n2;
-      const int ee = e0 + fe;
-      if (ee >= nElems || elem_problem(rk.eprob, ee) < 0) continue;
-      const int loc = face + 1, fnode = face_node<N>(loc, ab % n, ab / n);
-      const int sd = e2s[(ee * 6 + face) * 2] - 1, fl = e2s[(ee * 6 + face) * 2 + 1];
-      int p, q;
-      vol_to_side<N>(loc, fl, fnode % n, (fnode / n) % n, fnode / n2, p, q);
-      const size_t f = ((size_t)(sd * n + q) * n + p) * MV;
-      const double *F = (fl == 0) ? FluxM + f : FluxS + f;
-      const double sg = (fl == 0) ? L0 : -L0;
-#pragma unroll
-      for (int v = 0; v < MV; v++) s_face[fe][r * MV + v] = F[v] * sg;
+    for (int q = 0; q < 3; q++) {
+      m[q] = Mf[c * 3 + q];
+      m[3 + q] = Mg[c * 3 + q];
+      m[6 + q] = Mh[c * 3 + q];
     }
   }
-  __syncthreads();
-  for (int idx = tid; idx < EPB * n3; idx += T) {
-    const int el2 = idx / n3, node2 = idx - el2 * n3, e2 = e0 + el2;
-    if (e2 >= nElems) continue;
-    const int prob = elem_problem(rk.eprob, e2);
-    if (prob < 0) continue;
-    const int i2 = node2 % n, j2 = (node2 / n) % n, k2 = node2 / n2, l2 = Lds<N>::li(node2);
-    double tot[MV];
+  double fs[MV];  // the node's surface terms
 #pragma unroll
-    for (int v = 0; v < MV; v++) {
-      VR sd = MA_AT(el2, 0, v, l2);
-      sd = sd + MA_AT(el2, 1, v, l2);
-      sd = sd + MA_AT(el2, 2, v, l2);
-      tot[v] = double(sd);
-    }
-    if (PARA && MODE != VMODE_VOLINT) {  // VolInt_visc (volint.f90:228-271), formed by the lifting kernel
-      const double *uv = Uv + ((size_t)e2 * n3 + node2) * 7;
-#pragma unroll
-      for (int v = 1; v < 8; v++) tot[v] = tot[v] + uv[v - 1];
-    }
-    if (MODE != VMODE_VOLINT) {
-      const NodeFaces nf = node_faces<N>(i2, j2, k2);
-#pragma unroll
-      for (int t = 0; t < 3; t++) {
-        const int r = nf.get(t);
-        if (r < 0) continue;
-#pragma unroll
-        for (int v = 0; v < MV; v++) tot[v] = tot[v] + s_face[el2][r * MV + v];
-      }
-      const double msj = -sJ[(size_t)e2 * n3 + node2];
-#pragma unroll
-      for (int v = 0; v < MV; v++) tot[v] = tot[v] * msj;
-    }
-    const size_t o = ((size_t)e2 * n3 + node2) * MV;
-    if (MODE == VMODE_RK) {
-      const double bdt = rk.b * rk.st[prob].dt;
-#pragma unroll
-      for (int v = 0; v < MV; v++) {
-        const double ut = rk.first ? tot[v] : Uttmp[o + v] * (-rk.A) + tot[v];
-        Uttmp[o + v] = ut;
-        U[o + v] = U[o + v] + ut * bdt;
-      }
-    } else {
-#pragma unroll
-      for (int v = 0; v < MV; v++) Ut[o + v] = tot[v];
-    }
-  }
-#undef MF_AT
-#undef MM_AT
-#undef MA_AT
-}
-
-// The line form of the GLM-MHD volume kernel, used for the split-precision path: one thread
-// per (direction, element, line) evaluates each pair's flux once and keeps the n nodes' sums
-// in registers (in FP32 these fit at two waves per SIMD, and evaluating every pair once is
-// faster there than the node form above).  Same phases and sums otherwise.
-template <int N> struct MhdLineGeom;
-template <> struct MhdLineGeom<2> { static constexpr int EPB = 7, W = 64; };
-template <> struct MhdLineGeom<3> { static constexpr int EPB = 4, W = 64; };
-template <> struct MhdLineGeom<4> { static constexpr int EPB = 2, W = 64; };
-template <> struct MhdLineGeom<5> { static constexpr int EPB = 1, W = 64; };
-
-template <int N, int MODE, typename VR, bool PARA>
-__global__ void __launch_bounds__(3 * MhdLineGeom<N>::W)
-k_mhd_volume_line(double *__restrict__ U, const VR *__restrict__ Mf, const VR *__restrict__ Mg, const VR *__restrict__ Mh,
-             const double *__restrict__ sJ, const int *__restrict__ e2s, const double *__restrict__ FluxM,
-             const double *__restrict__ FluxS, const double *__restrict__ Uv, double *__restrict__ Ut,
-             double *__restrict__ Uttmp, RKArgs rk, int nElems, MhdArgs a, const DtState *__restrict__ st)
-{
-  constexpr int n = N + 1, n2 = n * n, n3 = n2 * n;
-  constexpr int EPB = MhdLineGeom<N>::EPB, W = MhdLineGeom<N>::W, NP = Lds<N>::NP;
-  static_assert(EPB * n2 <= W, "MHD volume launch geometry");
-  __shared__ VR s_f[EPB][MF_COUNT * NP];
-  __shared__ VR s_acc[EPB][MV * NP];
-  const Ops &op = c_ops[N];
-  const int tid = threadIdx.x, e0 = blockIdx.x * EPB;
-  const VR ch = VR(st->glm_ch), smu0 = VR(a.smu0), skm1 = VR(1.0 / (a.kappa - 1.0));
-
-  for (int idx = tid; idx < EPB * n3; idx += 3 * W) {
-    const int el = idx / n3, node = idx - el * n3, e = e0 + el;
-    if (e < nElems && elem_problem(rk.eprob, e) >= 0) {
-      const double *u = U + ((size_t)e * n3 + node) * MV;
-      double uu[MV], f[MF_COUNT];
-#pragma unroll
-      for (int v = 0; v < MV; v++) uu[v] = u[v];
-      mhd_node_fields(uu, a, f);
-      const int l = Lds<N>::li(node);
-#pragma unroll
-      for (int c = 0; c < MF_COUNT; c++) s_f[el][c * NP + l] = VR(f[c]);
-    }
-  }
-  __syncthreads();
-
-  const int dir = tid / W, lt = tid - dir * W;
-  const int el = lt / n2, line = lt - el * n2, e = e0 + el;
-  const bool active = (el < EPB) && (e < nElems) && elem_problem(rk.eprob, e) >= 0;
-  const int aa = line % n, bb = line / n;
-  int nodes[n], lds[n];
-#pragma unroll
-  for (int l = 0; l < n; l++) {
-    const int i = (dir == 0) ? l : aa, j = (dir == 1) ? l : (dir == 0 ? aa : bb), k = (dir == 2) ? l : bb;
-    nodes[l] = i + n * (j + n * k);
-    lds[l] = Lds<N>::li(i, j, k);
-  }
-  VR acc[n][MV], snc[n];
-#pragma unroll
-  for (int i = 0; i < n; i++) {
-    snc[i] = VR(0);
-#pragma unroll
-    for (int v = 0; v < MV; v++) acc[i][v] = VR(0);
-  }
-  if (active) {
-    const VR *M = (dir == 0) ? Mf : ((dir == 1) ? Mg : Mh);
-    VR m[n][3];
-#pragma unroll
-    for (int l = 0; l < n; l++) {
-      const VR *mp = M + ((size_t)e * n3 + nodes[l]) * 3;
-      m[l][0] = mp[0]; m[l][1] = mp[1]; m[l][2] = mp[2];
-    }
-#pragma unroll
-    for (int i = 0; i < n; i++)
-#pragma unroll
-      for (int l = i + 1; l < n; l++) {
-        VR fi[MF_COUNT], fl[MF_COUNT], F[MV];
-#pragma unroll
-        for (int c = 0; c < MF_COUNT; c++) { fi[c] = s_f[el][c * NP + lds[i]]; fl[c] = s_f[el][c * NP + lds[l]]; }
-        derigs_flux<VR>(fi, fl, m[i], m[l], ch, smu0, skm1, F);
-        const VR dil = OpsOf<VR>::ds(op, i, l), dli = OpsOf<VR>::ds(op, l, i);
-#pragma unroll
-        for (int v = 0; v < MV; v++) {
-          acc[i][v] += dil * F[v];
-          acc[l][v] += dli * F[v];
-        }
-        // Powell terms: B_l.{{m}} towards node i, B_i.{{m}} towards node l
-        const VR mb0 = VR(0.5) * (m[i][0] + m[l][0]), mb1 = VR(0.5) * (m[i][1] + m[l][1]),
-                 mb2 = VR(0.5) * (m[i][2] + m[l][2]);
-        snc[i] += dil * (mb0 * fl[MF_B1] + mb1 * fl[MF_B2] + mb2 * fl[MF_B3]);
-        snc[l] += dli * (mb0 * fi[MF_B1] + mb1 * fi[MF_B2] + mb2 * fi[MF_B3]);
-      }
-#pragma unroll
-    for (int i = 0; i < n; i++) {
-      const VR b1 = s_f[el][MF_B1 * NP + lds[i]], b2 = s_f[el][MF_B2 * NP + lds[i]], b3 = s_f[el][MF_B3 * NP + lds[i]];
-      const VR bhat = m[i][0] * b1 + m[i][1] * b2 + m[i][2] * b3;
-      const VR t = VR(0.5) * (bhat * VR(op.DsRow[i]) + snc[i]);
-      acc[i][1] += t * b1; acc[i][2] += t * b2; acc[i][3] += t * b3;
-      acc[i][4] += t * s_f[el][MF_VB * NP + lds[i]];
-      acc[i][5] += t * s_f[el][MF_V1 * NP + lds[i]];
-      acc[i][6] += t * s_f[el][MF_V2 * NP + lds[i]];
-      acc[i][7] += t * s_f[el][MF_V3 * NP + lds[i]];
-    }
-  }
-#pragma unroll
-  for (int d = 0; d < 3; d++) {
-    if (active && dir == d) {
-#pragma unroll
-      for (int l = 0; l < n; l++)
-#pragma unroll
-        for (int v = 0; v < MV; v++)
-          s_acc[el][v * NP + lds[l]] = (d == 0) ? acc[l][v] : s_acc[el][v * NP + lds[l]] + acc[l][v];
-    }
-    __syncthreads();
-  }
-
-  // the element's SurfInt terms +FluxM L0 (master) / -FluxS L0 (slave) into LDS in
-  // element-local face coordinates, one work item per face point
-  const double L0 = op.L0;
-  constexpr int NF = 6 * n2;
-  __shared__ double s_face[MODE != VMODE_VOLINT ? EPB : 1][MODE != VMODE_VOLINT ? NF * MV : 1];
+  for (int v = 0; v < MV; v++) fs[v] = 0.0;
   if (MODE != VMODE_VOLINT) {
-    for (int it = tid; it < EPB * NF; it += 3 * W) {
-      const int fe = it / NF, r = it - fe * NF, face = r / n2, ab = r - face * n2;
-      const int ee = e0 + fe;
+    // SurfInt terms +FluxM L0 (master) / -FluxS L0 (slave) in element-local face coordinates
+    const double L0 = op.L0;
+#pragma unroll
+    for (int it = tid; it < EPB * NF; it += T) {
+      const int fe = it / NF, r = it - fe * NF, face = r / n2, ab = r - face * n2, ee = e0 + fe;
       if (ee >= nElems || elem_problem(rk.eprob, ee) < 0) continue;
       const int loc = face + 1, fnode = face_node<N>(loc, ab % n, ab / n);
       const int sd = e2s[(ee * 6 + face) * 2] - 1, fl = e2s[(ee * 6 + face) * 2 + 1];
@@ -707,50 +462,117 @@ k_mhd_volume_line(double *__restrict__ U, const VR *__restrict__ Mf, const VR *_
       const double *F = (fl == 0) ? FluxM + f : FluxS + f;
       const double sg = (fl == 0) ? L0 : -L0;
 #pragma unroll
-      for (int v = 0; v < MV; v++) s_face[fe][r * MV + v] = F[v] * sg;
+      for (int v = 0; v < MV; v++) s_face[it * MV + v] = F[v] * sg;
     }
     __syncthreads();
-  }
-  for (int idx = tid; idx < EPB * n3; idx += 3 * W) {
-    const int el2 = idx / n3, node = idx - el2 * n3, e2 = e0 + el2;
-    if (e2 >= nElems) continue;
-    const int prob = elem_problem(rk.eprob, e2);
-    if (prob < 0) continue;
-    const int i = node % n, j = (node / n) % n, k = node / n2, l = Lds<N>::li(node);
-    double tot[MV];
-#pragma unroll
-    for (int v = 0; v < MV; v++) tot[v] = double(s_acc[el2][v * NP + l]);
-    if (PARA && MODE != VMODE_VOLINT) {  // VolInt_visc (volint.f90:228-271), formed by the lifting kernel
-      const double *uv = Uv + ((size_t)e2 * n3 + node) * 7;
-#pragma unroll
-      for (int v = 1; v < 8; v++) tot[v] = tot[v] + uv[v - 1];
-    }
-    if (MODE != VMODE_VOLINT) {
+    if (active) {
       const NodeFaces nf = node_faces<N>(i, j, k);
 #pragma unroll
       for (int t = 0; t < 3; t++) {
         const int r = nf.get(t);
         if (r < 0) continue;
 #pragma unroll
-        for (int v = 0; v < MV; v++) tot[v] = tot[v] + s_face[el2][r * MV + v];
+        for (int v = 0; v < MV; v++) fs[v] = fs[v] + s_face[(el * NF + r) * MV + v];
       }
-      const double msj = -sJ[(size_t)e2 * n3 + node];
-#pragma unroll
-      for (int v = 0; v < MV; v++) tot[v] = tot[v] * msj;
     }
-    const size_t o = ((size_t)e2 * n3 + node) * MV;
-    if (MODE == VMODE_RK) {
-      const double bdt = rk.b * rk.st[prob].dt;
+    __syncthreads();
+  }
+  VR own[MF_COUNT];
+  if (active) {
+    double f[MF_COUNT];
+    mhd_node_fields(u, a, f);
 #pragma unroll
-      for (int v = 0; v < MV; v++) {
-        const double ut = rk.first ? tot[v] : Uttmp[o + v] * (-rk.A) + tot[v];
-        Uttmp[o + v] = ut;
-        U[o + v] = U[o + v] + ut * bdt;
+    for (int q = 0; q < MF_COUNT; q++) {
+      own[q] = VR(f[q]);
+      if (q <= MF_LNBETA || q == MF_BB) s_f[mfs_slot(q) * NN + tid] = own[q];
+    }
+#pragma unroll
+    for (int q = 0; q < 9; q++) s_m[q * NN + tid] = VR(0.5) * m[q];
+    if (MODE == VMODE_RK) {
+#pragma unroll
+      for (int v = 1; v < 5; v++) s_u[(v - 1) * NN + tid] = u[v];
+      if (sizeof(VR) == 4) {
+#pragma unroll
+        for (int v = 4; v < MV; v++) s_u[v * NN + tid] = u[v == 4 ? 0 : v];
       }
+    }
+  }
+  __syncthreads();
+  if (!active) return;
+  const VR ch = VR(st->glm_ch), smu0 = VR(a.smu0), skm1 = VR(1.0 / (a.kappa - 1.0));
+  VR acc[MV], pw = VR(0);
+#pragma unroll
+  for (int v = 0; v < MV; v++) acc[v] = VR(0);
+  constexpr int PAIR_UNROLL = sizeof(VR) == 8 ? 2 : 1;  // FP64 by 1 spills, by 4 as fast; FP32 by 2: +2 %
+#pragma unroll 1
+  for (int d = 0; d < 3; d++) {
+    const int pos = (d == 0) ? i : ((d == 1) ? j : k), stride = (d == 0) ? 1 : ((d == 1) ? n : n2);
+    const VR *sm = s_m + 3 * d * NN;
+    const VR mo[3] = {sm[tid], sm[NN + tid], sm[2 * NN + tid]};
+#pragma unroll PAIR_UNROLL
+    for (int s = 1; s < n; s++) {
+      const int t2 = tid + (pos + s < n ? s : s - n) * stride;
+      VR nb[MF_COUNT], mn[3], F[MV], Bm;
+#pragma unroll
+      for (int q = 0; q < MF_COUNT; q++)
+        nb[q] = (q <= MF_LNBETA || q == MF_BB) ? s_f[mfs_slot(q) * NN + t2] : VR(0);
+#pragma unroll
+      for (int q = 0; q < 3; q++) mn[q] = sm[q * NN + t2];
+      derigs_flux2<VR>(own, nb, mo, mn, ch, smu0, skm1, F, Bm);
+      const VR ds = s_ds[s - 1][pos];
+#pragma unroll
+      for (int v = 0; v < MV; v++) acc[v] += ds * F[v];
+      pw += ds * Bm;
+    }
+    // the pair of the node with itself: its Dvolsurf row sum is what the others leave
+    pw += VR(op.DsRow[pos]) * (mo[0] * own[MF_B1] + mo[1] * own[MF_B2] + mo[2] * own[MF_B3]);
+  }
+  acc[1] += pw * own[MF_B1]; acc[2] += pw * own[MF_B2]; acc[3] += pw * own[MF_B3];
+  acc[4] += pw * own[MF_VB];
+  acc[5] += pw * own[MF_V1]; acc[6] += pw * own[MF_V2]; acc[7] += pw * own[MF_V3];
+  // the node pass: its loads first, its stores last and contiguous
+  double tt[MV], uv[7], sj = 0.0;
+  if (MODE == VMODE_RK) {
+#pragma unroll
+    for (int v = 0; v < MV; v++) tt[v] = rk.first ? 0.0 : Uttmp[c * MV + v];
+  }
+  if (MODE != VMODE_VOLINT) {
+    if (PARA) {
+#pragma unroll
+      for (int v = 0; v < 7; v++) uv[v] = Uv[c * 7 + v];
+    }
+    sj = sJ[c];
+  }
+  double tot[MV];
+#pragma unroll
+  for (int v = 0; v < MV; v++) tot[v] = double(acc[v]);
+  if (MODE != VMODE_VOLINT) {
+    if (PARA) {  // VolInt_visc (volint.f90:228-271), formed by the lifting kernel
+#pragma unroll
+      for (int v = 1; v < 8; v++) tot[v] = tot[v] + uv[v - 1];
+    }
+#pragma unroll
+    for (int v = 0; v < MV; v++) tot[v] = (tot[v] + fs[v]) * -sj;
+  }
+  if (MODE == VMODE_RK) {
+    const double bdt = rk.b * rk.st[prob].dt;
+#pragma unroll
+    for (int v = 1; v < 5; v++) u[v] = s_u[(v - 1) * NN + tid];
+    if (sizeof(VR) == 8) {  // the fields rho, B and psi are the state's own values
+      u[0] = own[MF_RHO]; u[5] = own[MF_B1]; u[6] = own[MF_B2]; u[7] = own[MF_B3]; u[8] = own[MF_PSI];
     } else {
 #pragma unroll
-      for (int v = 0; v < MV; v++) Ut[o + v] = tot[v];
+      for (int v = 4; v < MV; v++) u[v == 4 ? 0 : v] = s_u[v * NN + tid];
     }
+#pragma unroll
+    for (int v = 0; v < MV; v++) tt[v] = rk.first ? tot[v] : tt[v] * (-rk.A) + tot[v];
+#pragma unroll
+    for (int v = 0; v < MV; v++) Uttmp[c * MV + v] = tt[v];
+#pragma unroll
+    for (int v = 0; v < MV; v++) U[c * MV + v] = u[v] + tt[v] * bdt;
+  } else {
+#pragma unroll
+    for (int v = 0; v < MV; v++) Ut[c * MV + v] = tot[v];
   }
 }
 
