@@ -6,7 +6,7 @@
 //   nvse          : per side face point (nx, ny, nz, SurfElem)
 //   Flux          : nVar x (N+1)^2 x nSides (Flux_master * SurfElem; slave uses -Flux)
 //   Uv            : NVV x (N+1)^3 x nElems, weak-form viscous volume term (components 1..NVV)
-//   FvN           : NVV x 2 x (N+1)^2 x nSides, each side's face-normal viscous flux
+//   FvN           : NVV x (N+1)^2 x nSides x 2, each side's face-normal viscous flux
 //
 // Kernel roles per RHS (one LSERK stage):
 //   k_lifting  element-centric BR1 gradients -> viscous fluxes -> Uv, FvN (Navier-Stokes,
@@ -858,9 +858,9 @@ k_surface(const double *__restrict__ U, const double *__restrict__ FvN, const in
   if (ES) riemann_es<ES ? RS : 33>(UL, UR, nv, kappa, lam, F);
   else riemann<RS>(UL, UR, nv, kappa, F, lam);
   if (PARA) {  // BR1: mean of the two sides' normal viscous fluxes
-    const double *fn = FvN + (size_t)gid * 8;
+    const double *fm = FvN + (size_t)gid * 4, *fs = fm + (size_t)nSides * n2 * 4;
 #pragma unroll
-    for (int c = 0; c < 4; c++) F[c + 1] = F[c + 1] + 0.5 * (fn[c] + fn[4 + c]);
+    for (int c = 0; c < 4; c++) F[c + 1] = F[c + 1] + 0.5 * (fm[c] + fs[c]);
   }
   double *o = Flux + (size_t)gid * 5;
 #pragma unroll
@@ -1073,13 +1073,16 @@ template <int N> struct LiftGeom { static constexpr int EPB = (256 / ((N + 1) * 
 // vis_dir gives the NVV = 4 nonzero components (momentum, energy) of f a0 + g a1 + h a2.
 struct NsLift {
   static constexpr int NV = 5, NVV = 4;
-  double kappa, mu0, KappasPr;
-  __device__ __forceinline__ void entropy(const double *u, double *w) const { cons_to_entropy(u, kappa, w); }
-  __device__ __forceinline__ void grad_prim(const double *u, double *g) const { grad_entropy_to_prim(u, kappa, g); }
+  double kappa, skappaM1, mu0, KappasPr;
+  __device__ __forceinline__ void entropy(const double *u, double *w) const { cons_to_entropy(u, kappa, skappaM1, w); }
+  __device__ __forceinline__ void grad_prim(const double *u, double *g) const
+  {
+    grad_entropy_to_prim(u, kappa, skappaM1, g);
+  }
   __device__ __forceinline__ void fluxes(const double *u, const double *gx, const double *gy, const double *gz,
                                          double *fv) const
   {
-    diff_flux(u, gx, gy, gz, kappa, mu0, KappasPr, fv);
+    diff_flux(u, gx, gy, gz, kappa, skappaM1, mu0, KappasPr, fv);
   }
   __device__ __forceinline__ static void vis_dir(const double *s, double a0, double a1, double a2, double *o)
   {
@@ -1091,9 +1094,10 @@ struct NsLift {
 // Outputs of the lifting kernel's viscous form (OUT=1), per element and side:
 //   Uv(NVV, n^3, E)      weak-form viscous volume term sum_l D_hat(i,l) (f~, g~, h~)(l) of
 //                        VolInt_visc (volint.f90:228-271), components 1..NVV;
-//   FvN(NVV, 2, n^2, S)  n.(f, g, h) of each side's element at every face point (master
-//                        normal; [0] master, [1] slave), whose mean is the BR1 viscous
-//                        surface flux (riemann.f90:155-168).
+//   FvN(NVV, n^2, S, 2)  n.(f, g, h) of each side's element at every face point (master
+//                        normal; [0] master, [1] slave from fvSlave), whose mean is the BR1
+//                        viscous surface flux (riemann.f90:155-168).  Each half is written by
+//                        one element per side, n^2 NVV values in one piece.
 // The element's transformed fluxes pass through LDS: s_ft holds 3 NVV values per node.
 #ifndef FX_LIFT_WAVES
 #define FX_LIFT_WAVES 1
@@ -1115,7 +1119,7 @@ k_lifting(const double *__restrict__ U, const double *__restrict__ Mf, const dou
           const double4 *__restrict__ nvse, double *__restrict__ out0,
           double *__restrict__ out1, double *__restrict__ out2, const int *__restrict__ eprob,
           int nElems, EQ eq, double etaBR2, const double *__restrict__ Um, const double *__restrict__ LiftM,
-          double *__restrict__ GradM, int nMortar, DtFuse dtf)
+          double *__restrict__ GradM, int nMortar, DtFuse dtf, size_t fvSlave)
 {
   constexpr int n = N + 1, n2 = n * n, n3 = n2 * n, NV = EQ::NV, NVV = EQ::NVV;
   constexpr int EPB = LiftGeom<N>::EPB, NF = 6 * n2;  // face points per element
@@ -1137,6 +1141,7 @@ k_lifting(const double *__restrict__ U, const double *__restrict__ Mf, const dou
   auto SW = [](int x) { return (N == 3 && FX_LIFT_SWZ) ? (x ^ (((x >> 5) & 1) * 10)) : x; };
 #define LW(el_, v_, node_) s_u[el_][(v_) * n3 + SW(node_)]
   __shared__ int s_fpt[EPB][NF];  // 2 * face point ((s n + q) n + p) + (0 master, 1 slave)
+  auto fv_offset = [&](int code) { return (size_t)(code >> 1) * NVV + ((code & 1) ? fvSlave : 0); };
   const Ops &op = c_ops[N];
   const int tid = threadIdx.x;
   const int el = tid / n3, node = tid - el * n3;
@@ -1145,6 +1150,18 @@ k_lifting(const double *__restrict__ U, const double *__restrict__ Mf, const dou
   const int i = node % n, j = (node / n) % n, k = node / n2;
   const size_t c = (size_t)e * n3 + node;
   static_assert(!DT || (NV == 5 && OUT == 1), "CALCTIMESTEP in the Navier-Stokes stage lifting only");
+  // D and D_hat by column in LDS for the BR1 contractions without the matrix core: each lane reads
+  // its row's entry, which from constant memory is a vector load of its own (GLM-MHD N = 4, 24^3:
+  // 193 -> 178 us, Navier-Stokes N = 5: 44.6 -> 43 us; BR2 at N = 2 lost 1 us of 34 and keeps the
+  // constant memory)
+  constexpr bool LDSOP = N != 3 && LIFT == 1;
+  __shared__ double s_op[LDSOP ? 2 * n2 : 1];
+  if (LDSOP && tid < n2) {
+    s_op[tid] = op.D[tid % n][tid / n];
+    s_op[LDSOP ? n2 + tid : 0] = op.Dhat[tid % n][tid / n];
+  }
+  auto opD = [&](int r, int l) { return LDSOP ? s_op[l * n + r] : op.D[r][l]; };
+  auto opDhat = [&](int r, int l) { return LDSOP ? s_op[n2 + l * n + r] : op.Dhat[r][l]; };
   __shared__ unsigned long long s_dtl[DT ? EPB : 1][6];  // bit patterns of the element maxima
   __shared__ int s_dterr[DT ? EPB : 1];
   if (DT && tid < EPB * 7) {
@@ -1285,18 +1302,18 @@ k_lifting(const double *__restrict__ U, const double *__restrict__ Mf, const dou
     } else {
 #pragma unroll
       for (int v = 0; v < NV; v++) {
-        gxi[v] = op.D[i][0] * LW(el, v, 0 + n * (j + n * k));
-        geta[v] = op.D[j][0] * LW(el, v, i + n * (0 + n * k));
-        gzeta[v] = op.D[k][0] * LW(el, v, i + n * (j + n * 0));
+        gxi[v] = opD(i, 0) * LW(el, v, 0 + n * (j + n * k));
+        geta[v] = opD(j, 0) * LW(el, v, i + n * (0 + n * k));
+        gzeta[v] = opD(k, 0) * LW(el, v, i + n * (j + n * 0));
       }
       // not unrolled: all n NV LDS operands in flight at once would cost an occupancy level
 #pragma unroll 1
       for (int l = 1; l < n; l++)
 #pragma unroll
         for (int v = 0; v < NV; v++) {
-          gxi[v] = gxi[v] + op.D[i][l] * LW(el, v, l + n * (j + n * k));
-          geta[v] = geta[v] + op.D[j][l] * LW(el, v, i + n * (l + n * k));
-          gzeta[v] = gzeta[v] + op.D[k][l] * LW(el, v, i + n * (j + n * l));
+          gxi[v] = gxi[v] + opD(i, l) * LW(el, v, l + n * (j + n * k));
+          geta[v] = geta[v] + opD(j, l) * LW(el, v, i + n * (l + n * k));
+          gzeta[v] = gzeta[v] + opD(k, l) * LW(el, v, i + n * (j + n * l));
         }
     }
     const double *mf = PREM ? mreg : Mf + 3 * c, *mg = PREM ? mreg + 3 : Mg + 3 * c, *mh = PREM ? mreg + 6 : Mh + 3 * c;
@@ -1376,7 +1393,7 @@ k_lifting(const double *__restrict__ U, const double *__restrict__ Mf, const dou
           eq.grad_prim(u, fz);
           eq.fluxes(u, fx, fy, fz, fv);
           EQ::vis_dir(fv, nx, ny, nz, o);
-          double *dst = out1 + (size_t)s_fpt[el][r] * NVV;
+          double *dst = out1 + fv_offset(s_fpt[el][r]);
 #pragma unroll
           for (int v = 0; v < NVV; v++) dst[v] = o[v];
         }
@@ -1446,7 +1463,7 @@ k_lifting(const double *__restrict__ U, const double *__restrict__ Mf, const dou
       if (r < 0) continue;
       const double *d = &s_u[el][WSZ + r * (NV + 3)];
       EQ::vis_dir(fv, d[NV], d[NV + 1], d[NV + 2], o);
-      double *dst = out1 + (size_t)s_fpt[el][r] * NVV;
+      double *dst = out1 + fv_offset(s_fpt[el][r]);
 #pragma unroll
       for (int v = 0; v < NVV; v++) dst[v] = o[v];
     }
@@ -1505,7 +1522,7 @@ k_lifting(const double *__restrict__ U, const double *__restrict__ Mf, const dou
           const int code = s_fpt[el][r];
           const double4 g = nvse[code >> 1];
           EQ::vis_dir(fv, g.x, g.y, g.z, o);
-          double *dst = out1 + (size_t)code * NVV;
+          double *dst = out1 + fv_offset(code);
 #pragma unroll
           for (int v = 0; v < NVV; v++) dst[v] = o[v];
         }
@@ -1549,7 +1566,7 @@ k_lifting(const double *__restrict__ U, const double *__restrict__ Mf, const dou
       for (int v = 0; v < NVV; v++) uv[v] = 0.0;
 #pragma unroll 1
       for (int l = 0; l < n; l++) {
-        const double di = op.Dhat[i][l], dj = op.Dhat[j][l], dk = op.Dhat[k][l];
+        const double di = opDhat(i, l), dj = opDhat(j, l), dk = opDhat(k, l);
 #pragma unroll
         for (int v = 0; v < NVV; v++)
           uv[v] = uv[v] + di * s_u[el][v * n3 + SW(l + n * (j + n * k))] +
@@ -1638,7 +1655,7 @@ k_mortar_fv(const double *__restrict__ Um, const double *__restrict__ GradM, con
   eq.fluxes(u, gr, gr + NV, gr + 2 * NV, fv);
   const double4 g = nvse[fpt];
   EQ::vis_dir(fv, g.x, g.y, g.z, o);
-  double *dst = FvN + (2 * fpt) * NVV;
+  double *dst = FvN + fpt * NVV;
 #pragma unroll
   for (int v = 0; v < NVV; v++) dst[v] = o[v];
 }
@@ -1796,7 +1813,7 @@ k_entropy(const double *__restrict__ U, const double *__restrict__ Ut, const dou
     double el = -uu[0] * (log(p) - kappa * log(uu[0]));
     a = el * wv / sJ[gid];
     double w[5];
-    cons_to_entropy(uu, kappa, w);
+    cons_to_entropy(uu, kappa, 1.0 / km1, w);
     double s = 0.0;
 #pragma unroll
     for (int v = 0; v < 5; v++) s += w[v] * Ut[5 * gid + v];

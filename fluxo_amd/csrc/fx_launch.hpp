@@ -407,7 +407,8 @@ struct Batch {
   double *U = nullptr, *Ut = nullptr, *Uttmp = nullptr;
   double *Mf = nullptr, *Mg = nullptr, *Mh = nullptr, *sJ = nullptr;
   float *Mf32 = nullptr, *Mg32 = nullptr, *Mh32 = nullptr;  // split precision only
-  // viscous terms formed by the lifting kernel: Uv (NVV per node), FvN (2 NVV per face point)
+  // viscous terms formed by the lifting kernel: Uv (NVV per node), FvN (NVV per face
+  // point, the masters' values and after them the slaves')
   double *Flux = nullptr, *Uv = nullptr, *FvN = nullptr, *grad = nullptr;
   double4 *nvse = nullptr;
   int *e2s = nullptr, *s2e = nullptr;

@@ -180,22 +180,23 @@ void launch_lifting_l(const Batch &b, int out, const EQ &eq, const DtFuse *dtf)
   if (nb <= 0) return;
   const size_t nv = (size_t)EQ::NV * b.n3 * b.cfg.nElems;
   const DtFuse none{};
+  const size_t fvs = (size_t)b.cfg.nSides * b.n2 * EQ::NVV;  // FvN's slave half
   if (out == 0)
     hipLaunchKernelGGL((k_lifting<N, 0, EQ, LIFT>), dim3(nb), dim3(256), 0, b.stream, b.U, b.Mf, b.Mg, b.Mh, b.sJ,
                        b.ftab, b.nvse, b.grad, b.grad + nv, b.grad + 2 * nv, b.eprob, b.cfg.nElems, eq,
-                       b.cfg.etaBR2, b.Umort, b.LiftM, b.GradM, b.nMortar, none);
+                       b.cfg.etaBR2, b.Umort, b.LiftM, b.GradM, b.nMortar, none, fvs);
   else if constexpr (std::is_same<EQ, NsLift>::value) {
     if (dtf) {
       hipLaunchKernelGGL((k_lifting<N, 1, EQ, LIFT, true>), dim3(nb), dim3(256), 0, b.stream, b.U, b.Mf, b.Mg, b.Mh,
                          b.sJ, b.ftab, b.nvse, b.Uv, b.FvN, nullptr, b.eprob, b.cfg.nElems, eq, b.cfg.etaBR2,
-                         b.Umort, b.LiftM, b.GradM, b.nMortar, *dtf);
+                         b.Umort, b.LiftM, b.GradM, b.nMortar, *dtf, fvs);
       return;
     }
   }
   if (out != 0)
     hipLaunchKernelGGL((k_lifting<N, 1, EQ, LIFT>), dim3(nb), dim3(256), 0, b.stream, b.U, b.Mf, b.Mg, b.Mh, b.sJ,
                        b.ftab, b.nvse, b.Uv, b.FvN, nullptr, b.eprob, b.cfg.nElems, eq, b.cfg.etaBR2,
-                       b.Umort, b.LiftM, b.GradM, b.nMortar, none);
+                       b.Umort, b.LiftM, b.GradM, b.nMortar, none, fvs);
 }
 
 // Lifting (BR1 or BR2) on a mesh with mortars: U_Mortar of the state, the small sides' lifting
@@ -239,6 +240,7 @@ void launch_lifting_n(const Batch &b, int out, const DtFuse *dtf)
   if (b.mhd()) {
     MhdLift eq;
     eq.kappa = b.cfg.kappa;
+    eq.skappaM1 = 1.0 / (b.cfg.kappa - 1.0);
     eq.smu0 = 1.0 / b.cfg.mu_0;
     eq.mu = b.cfg.mu0;
     eq.etasmu0 = b.cfg.eta * eq.smu0;
@@ -248,6 +250,7 @@ void launch_lifting_n(const Batch &b, int out, const DtFuse *dtf)
   } else {
     NsLift eq;
     eq.kappa = b.cfg.kappa;
+    eq.skappaM1 = 1.0 / (b.cfg.kappa - 1.0);
     eq.mu0 = b.cfg.mu0;
     eq.KappasPr = b.cfg.kappa / b.cfg.Pr;
     if (b.nMortar > 0) launch_lifting_mortar<N>(b, out, eq, dtf);

@@ -137,7 +137,7 @@ __device__ __forceinline__ void mhd_visc_dir(const R *s, const R *a, R *o)
 // fluxes); g1 = f2, h1 = f3, h2 = g3, g5 = -f6, h5 = -f7, h6 = -g7, the rest vanish.
 struct MhdLift {
   static constexpr int NV = 9, NVV = 7;
-  double kappa, smu0, mu, etasmu0, KappasPr;
+  double kappa, skappaM1, smu0, mu, etasmu0, KappasPr;
   // components 1..7 of f a0 + g a1 + h a2
   __device__ __forceinline__ static void vis_dir(const double *s, double a0, double a1, double a2, double *o)
   {
@@ -147,50 +147,52 @@ struct MhdLift {
 #pragma unroll
     for (int v = 0; v < 7; v++) o[v] = t[v + 1];
   }
+  // 1/rho, velocity, |v|^2/2 and pressure of a state; the three functions below take them from the
+  // same expressions, which the lifting kernel then evaluates once per state (PrimState)
+  struct Prim {
+    double srho, u, v, w, v2s2, p;
+    __device__ __forceinline__ Prim(const double *c, double kappa, double smu0)
+    {
+      srho = 1.0 / c[0];
+      u = c[1] * srho; v = c[2] * srho; w = c[3] * srho;
+      v2s2 = 0.5 * (u * u + v * v + w * w);
+      const double b2 = c[5] * c[5] + c[6] * c[6] + c[7] * c[7] + c[8] * c[8];
+      p = (kappa - 1.0) * (c[4] - c[0] * v2s2 - 0.5 * smu0 * b2);
+    }
+  };
   __device__ __forceinline__ void entropy(const double *c, double *w) const
   {
-    const double km1 = kappa - 1.0, s2mu0 = 0.5 * smu0;
-    const double srho = 1.0 / c[0];
-    const double u = c[1] * srho, v = c[2] * srho, ww = c[3] * srho;
-    const double v2s2 = 0.5 * (u * u + v * v + ww * ww);
-    const double b2 = c[5] * c[5] + c[6] * c[6] + c[7] * c[7] + c[8] * c[8];
-    const double rho_sp = c[0] / (km1 * (c[4] - c[0] * v2s2 - s2mu0 * b2));
-    const double s = -log(rho_sp * pow(c[0], km1));
-    w[0] = (kappa - s) * (1.0 / km1) - rho_sp * v2s2;
-    w[1] = rho_sp * u;
-    w[2] = rho_sp * v;
-    w[3] = rho_sp * ww;
+    const Prim q(c, kappa, smu0);
+    const double rho_sp = c[0] / q.p;
+    const double s = -(log(rho_sp) + (kappa - 1.0) * log(c[0]));
+    w[0] = (kappa - s) * skappaM1 - rho_sp * q.v2s2;
+    w[1] = rho_sp * q.u;
+    w[2] = rho_sp * q.v;
+    w[3] = rho_sp * q.w;
     w[4] = -rho_sp;
 #pragma unroll
     for (int i = 5; i < NV; i++) w[i] = rho_sp * c[i];
   }
   __device__ __forceinline__ void grad_prim(const double *c, double *g) const
   {
-    const double km1 = kappa - 1.0, s2mu0 = 0.5 * smu0;
-    const double srho = 1.0 / c[0];
-    const double u = c[1] * srho, v = c[2] * srho, w = c[3] * srho;
-    const double ekin = 0.5 * (c[1] * u + c[2] * v + c[3] * w);
-    const double b2 = c[5] * c[5] + c[6] * c[6] + c[7] * c[7] + c[8] * c[8];
-    const double p = km1 * (c[4] - ekin - s2mu0 * b2);
-    const double rho_sp = c[0] / p, p_srho = p * srho;
+    const Prim q(c, kappa, smu0);
+    const double rho_sp = c[0] / q.p, p_srho = q.p * q.srho;
     const double g1 = g[0], g5 = g[4];
-    const double gu = p_srho * (g[1] + u * g5), gv = p_srho * (g[2] + v * g5), gw = p_srho * (g[3] + w * g5);
-    g[0] = c[0] * g1 - g5 * (ekin - p * (1.0 / km1)) + rho_sp * (c[1] * gu + c[2] * gv + c[3] * gw);
+    const double gu = p_srho * (g[1] + q.u * g5), gv = p_srho * (g[2] + q.v * g5), gw = p_srho * (g[3] + q.w * g5);
+    g[0] = c[0] * g1 - g5 * (c[0] * q.v2s2 - q.p * skappaM1) + rho_sp * (c[1] * gu + c[2] * gv + c[3] * gw);
     g[1] = gu;
     g[2] = gv;
     g[3] = gw;
-    g[4] = p_srho * (g[0] + p * g5);
+    g[4] = p_srho * (g[0] + q.p * g5);
 #pragma unroll
     for (int i = 5; i < NV; i++) g[i] = p_srho * (g[i] + c[i] * g5);
   }
   __device__ __forceinline__ void fluxes(const double *c, const double *gx, const double *gy, const double *gz,
                                          double *sv) const
   {
-    const double km1 = kappa - 1.0, skm1 = 1.0 / km1, s2mu0 = 0.5 * smu0, s23 = 2.0 / 3.0;
-    const double srho = 1.0 / c[0];
-    const double v1 = c[1] * srho, v2 = c[2] * srho, v3 = c[3] * srho;
-    const double b2 = c[5] * c[5] + c[6] * c[6] + c[7] * c[7] + c[8] * c[8];
-    const double p = km1 * (c[4] - 0.5 * (c[0] * (v1 * v1 + v2 * v2 + v3 * v3)) - s2mu0 * b2);
+    const double skm1 = skappaM1, s23 = 2.0 / 3.0;
+    const Prim q(c, kappa, smu0);
+    const double srho = q.srho, v1 = q.u, v2 = q.v, v3 = q.w, p = q.p;
     const double b1 = c[5], bb2 = c[6], b3 = c[7];
     const double divv = gx[1] + gy[2] + gz[3];
     const double lambda = mu * KappasPr;
@@ -322,9 +324,9 @@ k_mhd_surface(const double *__restrict__ U, const double *__restrict__ FvN, cons
     mhd_riemann_ec<RS>(UL, UR, nv, a, ch, Fm);
   }
   if (PARA) {  // BR1: mean of the two sides' normal diffusive fluxes
-    const double *fn = FvN + (size_t)gid * 14;
+    const double *fm = FvN + (size_t)gid * 7, *fs = fm + (size_t)nSides * n2 * 7;
 #pragma unroll
-    for (int v = 1; v < 8; v++) Fm[v] = Fm[v] + 0.5 * (fn[v - 1] + fn[6 + v]);
+    for (int v = 1; v < 8; v++) Fm[v] = Fm[v] + 0.5 * (fm[v - 1] + fs[v - 1]);
   }
 #pragma unroll
   for (int v = 0; v < MV; v++) Fs[v] = Fm[v];

@@ -733,52 +733,56 @@ __device__ __forceinline__ double face_lambda(const double *UL, const double *UR
 }
 
 // ConsToEntropy (navierstokes/equation_vars.f90:362-391); s = -ln(rho_sp*rho^(kappa-1))
+// 1/rho, velocity, |v|^2/2 and pressure of a state.  The lifting kernel forms entropy variables,
+// primitive gradients and viscous fluxes from one state: as the same expressions they are evaluated
+// once per state, with one division each for 1/rho and rho/p.
+struct PrimState {
+  double srho, v1, v2, v3, v2s2, p;
+  __device__ __forceinline__ PrimState(const double *U, double kappa)
+  {
+    srho = 1.0 / U[0];
+    v1 = U[1] * srho; v2 = U[2] * srho; v3 = U[3] * srho;
+    v2s2 = 0.5 * (v1 * v1 + v2 * v2 + v3 * v3);
+    p = (kappa - 1.0) * (U[4] - U[0] * v2s2);
+  }
+};
+
 // is evaluated as -(ln rho_sp + (kappa-1) ln rho).
-__device__ __forceinline__ void cons_to_entropy(const double *U, double kappa, double *w)
+__device__ __forceinline__ void cons_to_entropy(const double *U, double kappa, double skappaM1, double *w)
 {
-  double km1 = kappa - 1.0;
-  double srho = 1.0 / U[0];
-  double u = U[1] * srho, v = U[2] * srho, ww = U[3] * srho;
-  double v2s2 = 0.5 * (u * u + v * v + ww * ww);
-  double rho_sp = U[0] / (km1 * (U[4] - U[0] * v2s2));
-  double s = -(log(rho_sp) + km1 * log(U[0]));
-  w[0] = (kappa - s) / km1 - rho_sp * v2s2;
-  w[1] = rho_sp * u;
-  w[2] = rho_sp * v;
-  w[3] = rho_sp * ww;
+  const PrimState q(U, kappa);
+  const double rho_sp = U[0] / q.p;
+  const double s = -(log(rho_sp) + (kappa - 1.0) * log(U[0]));
+  w[0] = (kappa - s) * skappaM1 - rho_sp * q.v2s2;
+  w[1] = rho_sp * q.v1;
+  w[2] = rho_sp * q.v2;
+  w[3] = rho_sp * q.v3;
   w[4] = -rho_sp;
 }
 
 // ConvertToGradPrimVec for entropy-variable lifting (equation_vars.f90:571-647).
-__device__ __forceinline__ void grad_entropy_to_prim(const double *U, double kappa, double *g)
+__device__ __forceinline__ void grad_entropy_to_prim(const double *U, double kappa, double skappaM1, double *g)
 {
-  double km1 = kappa - 1.0, skm1 = 1.0 / km1;
-  double srho = 1.0 / U[0];
-  double u = U[1] * srho, v = U[2] * srho, w = U[3] * srho;
-  double ekin = 0.5 * (U[1] * u + U[2] * v + U[3] * w);
-  double p = km1 * (U[4] - ekin);
-  double rho_sp = U[0] / p;
-  double p_srho = p * srho;
-  double g1 = g[0];
-  double gu = p_srho * (g[1] + u * g[4]);
-  double gv = p_srho * (g[2] + v * g[4]);
-  double gw = p_srho * (g[3] + w * g[4]);
-  double g5 = g[4];
-  g[0] = U[0] * g1 - g5 * (ekin - p * skm1) + rho_sp * (U[1] * gu + U[2] * gv + U[3] * gw);
+  const PrimState q(U, kappa);
+  const double rho_sp = U[0] / q.p, p_srho = q.p * q.srho;
+  const double g1 = g[0], g5 = g[4];
+  const double gu = p_srho * (g[1] + q.v1 * g5);
+  const double gv = p_srho * (g[2] + q.v2 * g5);
+  const double gw = p_srho * (g[3] + q.v3 * g5);
+  g[0] = U[0] * g1 - g5 * (U[0] * q.v2s2 - q.p * skappaM1) + rho_sp * (U[1] * gu + U[2] * gv + U[3] * gw);
   g[1] = gu; g[2] = gv; g[3] = gw;
-  g[4] = p_srho * (g[0] + p * g5);
+  g[4] = p_srho * (g[0] + q.p * g5);
 }
 
 // EvalDiffFlux3D with constant viscosity (flux.f90:407-517): Cartesian viscous fluxes
 // f, g, h; component 0 (mass) is identically zero and omitted: out[d*4 + (v-1)].
 __device__ __forceinline__ void diff_flux(const double *U, const double *gx, const double *gy,
-                                          const double *gz, double kappa, double mu0,
+                                          const double *gz, double kappa, double skm1, double mu0,
                                           double KappasPr, double *out)
 {
-  const double km1 = kappa - 1.0, skm1 = 1.0 / km1, s23 = 2.0 / 3.0;
-  double srho = 1.0 / U[0];
-  double v1 = U[1] * srho, v2 = U[2] * srho, v3 = U[3] * srho;
-  double p = km1 * (U[4] - 0.5 * (U[1] * v1 + U[2] * v2 + U[3] * v3));
+  const double s23 = 2.0 / 3.0;
+  const PrimState q(U, kappa);
+  const double srho = q.srho, v1 = q.v1, v2 = q.v2, v3 = q.v3, p = q.p;
   double muS = mu0, lambda = muS * KappasPr;
   double divv = gx[1] + gy[2] + gz[3];
   double cTx = skm1 * srho * (gx[4] - srho * p * gx[0]);
