@@ -13,6 +13,7 @@
 #include "fx_kernels.hpp"
 #include "fx_launch.hpp"
 #include "fx_analyze.hpp"
+#include "fx_hostcopy.hpp"
 
 namespace fx {
 
@@ -51,9 +52,32 @@ struct fx_ctx {
   bool mesh_ok = false, state_ok = false;
   hipGraphExec_t graph = nullptr;
   double graph_cfl = -1.0, graph_dfl = -1.0;
+  std::shared_ptr<HostCopy> copier;  // workers of large host copies, from the first one on
 };
 
 namespace {
+
+// A copy between the caller's host array and device memory, complete on return (ordered behind the
+// work queued on the context's stream).
+int host_copy(fx_ctx *c, void *dst, const void *src, size_t bytes, hipMemcpyKind kind)
+{
+  hipStream_t st = c->b.stream;
+  const bool up = kind == hipMemcpyHostToDevice;
+  if (bytes >= HostCopy::MIN_BYTES && pageable_host(up ? src : dst)) {
+    if (!c->copier) {
+      int dev = -1;
+      if (hipGetDevice(&dev) == hipSuccess) c->copier = HostCopy::get(dev);
+    }
+    hipError_t e = hipSuccess;
+    if (c->copier && c->copier->copy(dst, src, bytes, up, st, &e)) {
+      HIPCHK(e);
+      return FX_OK;
+    }
+  }
+  HIPCHK(hipMemcpyAsync(dst, src, bytes, kind, st));
+  HIPCHK(hipStreamSynchronize(st));
+  return FX_OK;
+}
 
 size_t vol_doubles(const fx_config &c) { size_t n = c.N + 1; return (size_t)c.nVar * n * n * n * c.nElems; }
 
@@ -300,8 +324,8 @@ int fx_mesh_upload(fx_ctx *c, const fx_mesh *m)
 int fx_state_upload(fx_ctx *c, const double *U)
 {
   if (!c || !U) return set_err(FX_EINVAL, "null argument");
-  HIPCHK(hipMemcpyAsync(c->b.U, U, vol_doubles(c->b.cfg) * 8, hipMemcpyHostToDevice, c->b.stream));
-  HIPCHK(hipStreamSynchronize(c->b.stream));
+  const int rc = host_copy(c, c->b.U, U, vol_doubles(c->b.cfg) * 8, hipMemcpyHostToDevice);
+  if (rc) return rc;
   c->state_ok = true;
   return FX_OK;
 }
@@ -309,17 +333,13 @@ int fx_state_upload(fx_ctx *c, const double *U)
 int fx_state_download(fx_ctx *c, double *U)
 {
   if (!c || !U) return set_err(FX_EINVAL, "null argument");
-  HIPCHK(hipMemcpyAsync(U, c->b.U, vol_doubles(c->b.cfg) * 8, hipMemcpyDeviceToHost, c->b.stream));
-  HIPCHK(hipStreamSynchronize(c->b.stream));
-  return FX_OK;
+  return host_copy(c, U, c->b.U, vol_doubles(c->b.cfg) * 8, hipMemcpyDeviceToHost);
 }
 
 int fx_ut_download(fx_ctx *c, double *Ut)
 {
   if (!c || !Ut) return set_err(FX_EINVAL, "null argument");
-  HIPCHK(hipMemcpyAsync(Ut, c->b.Ut, vol_doubles(c->b.cfg) * 8, hipMemcpyDeviceToHost, c->b.stream));
-  HIPCHK(hipStreamSynchronize(c->b.stream));
-  return FX_OK;
+  return host_copy(c, Ut, c->b.Ut, vol_doubles(c->b.cfg) * 8, hipMemcpyDeviceToHost);
 }
 
 static int ready(fx_ctx *c)

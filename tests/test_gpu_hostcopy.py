@@ -1,0 +1,63 @@
+"""Host transfers of a context (fx_state_upload / fx_state_download): bytes unchanged at sizes around
+the threshold of the staged copy and around its chunks, from read-only and from new arrays, and with
+several contexts transferring at once from threads of their own."""
+import threading
+
+import numpy as np
+import pytest
+
+from fluxo_amd.mesh import box_mesh
+from fluxo_amd.native import Engine
+
+pytestmark = pytest.mark.gpu
+
+NODE_BYTES = 64 * 40  # an element at N = 3
+MIB = 1 << 20
+
+
+def context(elements):
+    m = box_mesh((elements, 1, 1), 3, length=(float(elements), 1.0, 1.0))
+    return Engine(m)
+
+
+def random_state(e, seed):
+    U = np.random.default_rng(seed).standard_normal(e.shape())
+    U.setflags(write=False)
+    return U
+
+
+@pytest.mark.parametrize("nbytes", [64 << 10, 4 * MIB, 8 * MIB, 33 * MIB])
+@pytest.mark.parametrize("step", [0, 1])
+def test_state_round_trip(nbytes, step):
+    e = context(nbytes // NODE_BYTES + step)  # the last size below and the first above
+    for seed in (1, 2):
+        U = random_state(e, seed)
+        e.upload(U)
+        assert np.array_equal(e.download(), U)
+    e.close()
+
+
+def test_contexts_transfer_at_once():
+    es = [context(6000 + 7 * i) for i in range(3)]
+    bad = []
+
+    def work(e, seed):
+        for r in range(4):
+            U = random_state(e, 10 * seed + r)
+            e.upload(U)
+            if not np.array_equal(e.download(), U):
+                bad.append((seed, r))
+
+    th = [threading.Thread(target=work, args=(e, i)) for i, e in enumerate(es)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert not bad
+    for e in es:
+        e.close()
+    e = context(6000)  # the workers are made again after the last context gave them back
+    U = random_state(e, 99)
+    e.upload(U)
+    assert np.array_equal(e.download(), U)
+    e.close()
