@@ -1714,6 +1714,36 @@ k_calc_dt(const double *__restrict__ U, const double *__restrict__ Mf, const dou
 }
 
 #ifdef FX_KERNEL_HOME  // non-template kernels: compiled in one unit only
+// Minimum and maximum error code of the entries i0, i0 + T, ... below i1 (NaN entries skipped: a
+// comparison with NaN is false).  DTR entries are loaded ahead of the first comparison: at one
+// load's latency per entry the one-block reduction of 64,000 elements took 24 us, now 14 us.
+constexpr int DTR = 8;
+template <int T>
+__device__ __forceinline__ void dt_minimum(const double *__restrict__ dt, const int *__restrict__ err, int i0, int i1,
+                                           double &m, int &er)
+{
+  int i = i0;
+  for (; i + (DTR - 1) * T < i1; i += DTR * T) {
+    double d[DTR];
+    int r[DTR];
+#pragma unroll
+    for (int q = 0; q < DTR; q++) {
+      d[q] = dt[i + q * T];
+      r[q] = err ? err[i + q * T] : 0;
+    }
+#pragma unroll
+    for (int q = 0; q < DTR; q++) {
+      if (d[q] < m) m = d[q];
+      er = max(er, r[q]);
+    }
+  }
+  for (; i < i1; i += T) {
+    const double d = dt[i];
+    if (d < m) m = d;
+    if (err) er = max(er, err[i]);
+  }
+}
+
 // Minimum of dtElem (NaN entries skipped) and maximum error code, one block, fixed order.
 __global__ void __launch_bounds__(1024)
 k_dt_reduce(const double *__restrict__ dtElem, const int *__restrict__ errElem, int nElems, DtState *st,
@@ -1724,11 +1754,7 @@ k_dt_reduce(const double *__restrict__ dtElem, const int *__restrict__ errElem, 
   const int tid = threadIdx.x;
   double m = 1.79e308;
   int er = 0;
-  for (int e = tid; e < nElems; e += 1024) {
-    const double d = dtElem[e];
-    if (d < m) m = d;
-    er = max(er, errElem[e]);
-  }
+  dt_minimum<1024>(dtElem, errElem, tid, nElems, m, er);
   s_dt[tid] = m;
   s_er[tid] = er;
   __syncthreads();
@@ -1763,11 +1789,7 @@ k_dt_reduce_seg(const double *__restrict__ dtElem, const int *__restrict__ errEl
   if (ne <= 0) return;
   double m = 1.79e308;
   int er = 0;
-  for (int e = e0 + tid; e < e0 + ne; e += 256) {
-    const double d = dtElem[e];
-    if (d < m) m = d;
-    er = max(er, errElem[e]);
-  }
+  dt_minimum<256>(dtElem, errElem, e0 + tid, e0 + ne, m, er);
   s_dt[tid] = m;
   s_er[tid] = er;
   __syncthreads();

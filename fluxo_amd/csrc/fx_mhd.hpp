@@ -662,12 +662,8 @@ k_mhd_dt_reduce(const double *__restrict__ dtElem, const double *__restrict__ dt
   const int tid = threadIdx.x;
   double m = 1.79e308, mc = 1.79e308;
   int er = 0;
-  for (int e = tid; e < nElems; e += 1024) {
-    const double d = dtElem[e], dc = dtch1Elem[e];
-    if (d < m) m = d;
-    if (dc < mc) mc = dc;
-    er = max(er, errElem[e]);
-  }
+  dt_minimum<1024>(dtElem, errElem, tid, nElems, m, er);
+  dt_minimum<1024>(dtch1Elem, nullptr, tid, nElems, mc, er);
   s_dt[tid] = m; s_c[tid] = mc; s_er[tid] = er;
   __syncthreads();
   for (int stp = 512; stp > 0; stp >>= 1) {
