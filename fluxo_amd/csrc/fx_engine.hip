@@ -3,6 +3,7 @@
 // layer (fx_launch.hpp) and the batched server (fx_server.hpp) are compiled with it.
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <mutex>
 #include <vector>
@@ -864,10 +865,14 @@ int scratch_ptr(unsigned char **out)
   return FX_OK;
 }
 
-// Scratch layout of one call, each part 256-byte aligned; returns the bytes needed.
+// Scratch layout of one call, each part 256-byte aligned; returns the bytes needed.  The check's
+// result comes first, where no other layout puts anything: it holds the number of the last call
+// whose connectivity was found invalid (numbers grow, so an older one says nothing; a newer one, of a
+// call that overlaps this one, refuses this one too).
 struct NoallocLayout {
-  size_t nvse = 0, ftab = 0, flux = 0, uv = 0, fvn = 0, alpha = 0, alpha2 = 0, ffv = 0, flag = 0, total = 0;
+  size_t flag = 0, nvse = 0, ftab = 0, flux = 0, uv = 0, fvn = 0, alpha = 0, alpha2 = 0, ffv = 0, total = 0;
 };
+std::atomic<unsigned long long> g_noalloc_calls{0};
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 NoallocLayout noalloc_layout(const fx_config &c)
 {
@@ -875,6 +880,7 @@ NoallocLayout noalloc_layout(const fx_config &c)
   NoallocLayout L;
   size_t o = 0;
   auto take = [&](size_t &at, size_t bytes) { at = o; o += align256(bytes); };
+  take(L.flag, sizeof(unsigned long long));
   take(L.nvse, nf * sizeof(double4));
   take(L.flux, 5 * nf * 8);
   if (c.parabolic) {
@@ -887,17 +893,19 @@ NoallocLayout noalloc_layout(const fx_config &c)
     take(L.alpha2, (size_t)c.nElems * 8);
     take(L.ffv, 5 * n3E * 8);
   }
-  take(L.flag, sizeof(int));
   L.total = o;
   return L;
 }
 
-__global__ void k_noalloc_flag_clear(int *flag) { flag[0] = 0; }
-
 // Device-side form of check_connectivity: every index the kernels derive from the caller's
-// ElemToSide / SideToElem must stay inside the mesh; any violation sets *flag.
+// ElemToSide / SideToElem must stay inside the mesh; any violation sets *flag to this call's
+// number.  In the same launch (nx, ny, nz, SurfElem) of the nf face points are packed into the layout
+// the kernels read, which needs no connectivity.  (One launch instead of three with the clearing of
+// the flag; the call at 8^3 elements, N = 3, took 38 us of which the host's launches bound.)
 __global__ void k_noalloc_check(const int *__restrict__ e2s, const int *__restrict__ s2e, int E, int S,
-                                int *__restrict__ flag)
+                                unsigned long long *__restrict__ flag, unsigned long long call,
+                                const double *__restrict__ nv, const double *__restrict__ se,
+                                double4 *__restrict__ nvse, long long nf)
 {
   const long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   int bad = 0;
@@ -916,15 +924,8 @@ __global__ void k_noalloc_check(const int *__restrict__ e2s, const int *__restri
     const int *a = e2s + 2 * (size_t)(g - S);
     if (a[0] < 1 || a[0] > S || a[1] < 0 || a[1] > 4) bad = 1;
   }
-  if (bad) atomicOr(flag, 1);
-}
-
-// (nx, ny, nz, SurfElem) per face point, the layout the kernels read
-__global__ void k_noalloc_pack_nvse(const double *__restrict__ nv, const double *__restrict__ se,
-                                    double4 *__restrict__ out, long long nf)
-{
-  const long long f = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (f < nf) out[f] = make_double4(nv[3 * f], nv[3 * f + 1], nv[3 * f + 2], se[f]);
+  if (bad) atomicMax(flag, call);
+  if (g < nf) nvse[g] = make_double4(nv[3 * g], nv[3 * g + 1], nv[3 * g + 2], se[g]);
 }
 
 }  // namespace
@@ -960,17 +961,20 @@ int fx_rhs_noalloc(const fx_config *cfg, const fx_mesh *mesh, const double *U, d
   if ((rc = scratch_ptr(&sp))) return rc;
   if ((rc = ensure_ops(cfg->N))) return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  int *flag = reinterpret_cast<int *>(sp + L.flag);
+  unsigned long long *flag = reinterpret_cast<unsigned long long *>(sp + L.flag);
+  const unsigned long long call = g_noalloc_calls.fetch_add(1) + 1;
+  double4 *nvse = reinterpret_cast<double4 *>(sp + L.nvse);
   // connectivity check on the device, read back before any kernel indexes through it
-  hipLaunchKernelGGL(k_noalloc_flag_clear, dim3(1), dim3(1), 0, st, flag);
-  const long long nchk = (long long)cfg->nSides + 6LL * cfg->nElems;
+  const long long nf = (long long)(cfg->N + 1) * (cfg->N + 1) * cfg->nSides;
+  const long long nchk = std::max((long long)cfg->nSides + 6LL * cfg->nElems, nf);
   hipLaunchKernelGGL(k_noalloc_check, dim3((unsigned)((nchk + 255) / 256)), dim3(256), 0, st,
-                     (const int *)mesh->ElemToSide, (const int *)mesh->SideToElem, cfg->nElems, cfg->nSides, flag);
+                     (const int *)mesh->ElemToSide, (const int *)mesh->SideToElem, cfg->nElems, cfg->nSides, flag,
+                     call, mesh->NormVec, mesh->SurfElem, nvse, nf);
   HIPCHK(hipGetLastError());
-  int hflag = 0;
-  HIPCHK(hipMemcpyAsync(&hflag, flag, sizeof(int), hipMemcpyDeviceToHost, st));
+  unsigned long long hflag = 0;
+  HIPCHK(hipMemcpyAsync(&hflag, flag, sizeof(hflag), hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
-  if (hflag) return set_err(FX_EINVAL, "fx_rhs_noalloc: ElemToSide / SideToElem invalid (only inner conforming "
+  if (hflag >= call) return set_err(FX_EINVAL, "fx_rhs_noalloc: ElemToSide / SideToElem invalid (only inner conforming "
                                        "sides are supported)");
   Batch b;
   b.cfg = *cfg;
@@ -984,7 +988,7 @@ int fx_rhs_noalloc(const fx_config *cfg, const fx_mesh *mesh, const double *U, d
   b.sJ = const_cast<double *>(mesh->sJ);
   b.e2s = const_cast<int *>(mesh->ElemToSide);
   b.s2e = const_cast<int *>(mesh->SideToElem);
-  b.nvse = reinterpret_cast<double4 *>(sp + L.nvse);
+  b.nvse = nvse;
   b.Flux = reinterpret_cast<double *>(sp + L.flux);
   if (cfg->parabolic) {
     b.ftab = reinterpret_cast<int2 *>(sp + L.ftab);
@@ -996,9 +1000,6 @@ int fx_rhs_noalloc(const fx_config *cfg, const fx_mesh *mesh, const double *U, d
     b.alpha2 = reinterpret_cast<double *>(sp + L.alpha2);
     b.Ffv = reinterpret_cast<double *>(sp + L.ffv);
   }
-  const long long nf = (long long)b.n2 * cfg->nSides;
-  hipLaunchKernelGGL(k_noalloc_pack_nvse, dim3((unsigned)((nf + 255) / 256)), dim3(256), 0, st, mesh->NormVec,
-                     mesh->SurfElem, b.nvse, nf);
   if (cfg->parabolic) FX_DISPATCH_N(b.cfg.N, launch_face_table_n, b, 0, cfg->nElems);
   RKArgs rk{};
   q_stage(b, VMODE_RHS, rk);
