@@ -53,32 +53,10 @@ struct fx_ctx {
   bool mesh_ok = false, state_ok = false;
   hipGraphExec_t graph = nullptr;
   double graph_cfl = -1.0, graph_dfl = -1.0;
-  std::shared_ptr<HostCopy> copier;  // workers of large host copies, from the first one on
+  HostTransfers host;  // state uploads and downloads
 };
 
 namespace {
-
-// A copy between the caller's host array and device memory, complete on return (ordered behind the
-// work queued on the context's stream).
-int host_copy(fx_ctx *c, void *dst, const void *src, size_t bytes, hipMemcpyKind kind)
-{
-  hipStream_t st = c->b.stream;
-  const bool up = kind == hipMemcpyHostToDevice;
-  if (bytes >= HostCopy::MIN_BYTES && pageable_host(up ? src : dst)) {
-    if (!c->copier) {
-      int dev = -1;
-      if (hipGetDevice(&dev) == hipSuccess) c->copier = HostCopy::get(dev);
-    }
-    hipError_t e = hipSuccess;
-    if (c->copier && c->copier->copy(dst, src, bytes, up, st, &e)) {
-      HIPCHK(e);
-      return FX_OK;
-    }
-  }
-  HIPCHK(hipMemcpyAsync(dst, src, bytes, kind, st));
-  HIPCHK(hipStreamSynchronize(st));
-  return FX_OK;
-}
 
 size_t vol_doubles(const fx_config &c) { size_t n = c.N + 1; return (size_t)c.nVar * n * n * n * c.nElems; }
 
@@ -178,6 +156,7 @@ int fx_ctx_create(const fx_config *cfg, fx_ctx **out)
     return e == hipErrorOutOfMemory ? FX_ENOMEM : FX_EHIP;
   };
   hipError_t e;
+  if ((e = hipGetDevice(&c->host.device)) != hipSuccess) return fail(e, "device");
   if ((e = hipStreamCreateWithFlags(&b.stream, hipStreamNonBlocking)) != hipSuccess) return fail(e, "stream");
 #define ALLOC(p, bytes)                                               \
   if ((e = hipMalloc((void **)&(p), (bytes))) != hipSuccess) return fail(e, "hipMalloc " #p);
@@ -325,8 +304,7 @@ int fx_mesh_upload(fx_ctx *c, const fx_mesh *m)
 int fx_state_upload(fx_ctx *c, const double *U)
 {
   if (!c || !U) return set_err(FX_EINVAL, "null argument");
-  const int rc = host_copy(c, c->b.U, U, vol_doubles(c->b.cfg) * 8, hipMemcpyHostToDevice);
-  if (rc) return rc;
+  HIPCHK(c->host.copy(c->b.U, U, vol_doubles(c->b.cfg) * 8, hipMemcpyHostToDevice, c->b.stream));
   c->state_ok = true;
   return FX_OK;
 }
@@ -334,13 +312,15 @@ int fx_state_upload(fx_ctx *c, const double *U)
 int fx_state_download(fx_ctx *c, double *U)
 {
   if (!c || !U) return set_err(FX_EINVAL, "null argument");
-  return host_copy(c, U, c->b.U, vol_doubles(c->b.cfg) * 8, hipMemcpyDeviceToHost);
+  HIPCHK(c->host.copy(U, c->b.U, vol_doubles(c->b.cfg) * 8, hipMemcpyDeviceToHost, c->b.stream));
+  return FX_OK;
 }
 
 int fx_ut_download(fx_ctx *c, double *Ut)
 {
   if (!c || !Ut) return set_err(FX_EINVAL, "null argument");
-  return host_copy(c, Ut, c->b.Ut, vol_doubles(c->b.cfg) * 8, hipMemcpyDeviceToHost);
+  HIPCHK(c->host.copy(Ut, c->b.Ut, vol_doubles(c->b.cfg) * 8, hipMemcpyDeviceToHost, c->b.stream));
+  return FX_OK;
 }
 
 static int ready(fx_ctx *c)

@@ -109,9 +109,23 @@ class HostCopy {
     ~Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&m); }
   };
 
+  // The calls of a scope on a device; the caller's current device afterwards.
+  struct OnDevice {
+    int prev = -1;
+    explicit OnDevice(int dev)
+    {
+      if (hipGetDevice(&prev) != hipSuccess || prev == dev || hipSetDevice(dev) != hipSuccess) prev = -1;
+    }
+    ~OnDevice()
+    {
+      if (prev >= 0) (void)hipSetDevice(prev);
+    }
+  };
+
   bool start()
   {
     Relaxed relaxed;
+    OnDevice here(dev_);  // an event can be recorded on its own device's streams only
     for (Slot &s : slot_)
       if (hipHostMalloc(&s.p, CHUNK, hipHostMallocDefault) != hipSuccess ||
           hipEventCreateWithFlags(&s.ev, hipEventDisableTiming) != hipSuccess) {
@@ -217,5 +231,29 @@ inline bool pageable_host(const void *p)
   }
   return a.type == hipMemoryTypeUnregistered;
 }
+
+// The transfers of one context: through the workers of the context's own device, whichever device
+// the calling thread has current, or by the plain copy.
+class HostTransfers {
+ public:
+  int device = -1;  // of the context's stream and memory
+
+  // A copy between the caller's host array and device memory, complete on return (ordered behind
+  // the work queued on the stream).
+  hipError_t copy(void *dst, const void *src, size_t bytes, hipMemcpyKind kind, hipStream_t stream) noexcept
+  {
+    const bool up = kind == hipMemcpyHostToDevice;
+    if (bytes >= HostCopy::MIN_BYTES && pageable_host(up ? src : dst)) {
+      if (!workers_) workers_ = HostCopy::get(device);
+      hipError_t e = hipSuccess;
+      if (workers_ && workers_->copy(dst, src, bytes, up, stream, &e)) return e;
+    }
+    const hipError_t e = hipMemcpyAsync(dst, src, bytes, kind, stream);
+    return e != hipSuccess ? e : hipStreamSynchronize(stream);
+  }
+
+ private:
+  std::shared_ptr<HostCopy> workers_;  // from the first large transfer on
+};
 
 }  // namespace fx

@@ -1,0 +1,57 @@
+// Checks of HostTransfers (fx_hostcopy.hpp) against the HIP calls of hip/hip_runtime.h beside this
+// file; the check to run is the argument.
+#include <cstdio>
+#include <string>
+#include <vector>
+
+#include "fx_hostcopy.hpp"
+
+using fx::HostTransfers;
+
+namespace {
+
+constexpr size_t MIB = (size_t)1 << 20;
+
+#define REQUIRE(x)                                                            \
+  do {                                                                        \
+    if (!(x)) {                                                               \
+      std::printf("line %d: %s\n", __LINE__, #x);                             \
+      return 1;                                                               \
+    }                                                                         \
+  } while (0)
+
+// up and down through a context's transfers: the bytes come back
+bool round_trip(HostTransfers &t, fakeStream &st, size_t bytes)
+{
+  std::vector<char> a(bytes), dev(bytes), b(bytes);
+  for (size_t i = 0; i < bytes; i += 511) a[i] = (char)(i * 2654435761u >> 7);
+  return t.copy(dev.data(), a.data(), bytes, hipMemcpyHostToDevice, &st) == hipSuccess &&
+         t.copy(b.data(), dev.data(), bytes, hipMemcpyDeviceToHost, &st) == hipSuccess && a == b;
+}
+
+// a context's transfers while its device is not the calling thread's current one
+int other_device()
+{
+  for (int current : {0, 1, 2}) {
+    fake::current = current;
+    for (int device : {0, 1}) {
+      HostTransfers t;
+      t.device = device;
+      fakeStream st{device};
+      for (int r = 0; r < 2; r++) REQUIRE(round_trip(t, st, 80 * MIB + 12345));
+      REQUIRE(fake::current == current);
+    }
+  }
+  REQUIRE(fake::staged > 0 && fake::pinned == 0);
+  return 0;
+}
+
+}  // namespace
+
+int main(int, char **argv)
+{
+  const std::string check = argv[1];
+  if (check == "other_device") return other_device();
+  std::printf("no check %s\n", argv[1]);
+  return 2;
+}
