@@ -8,10 +8,15 @@
 // (Pinned copies run at 57 GB/s here.)  Chunks of 1 and 2 MiB: every copy costs about 35 us of
 // its own, 84 MB up in 2.75 and 2.15 ms; 8 MiB loses on small transfers; 8 workers gain nothing.
 //
-// The workers and their pinned chunks (32 MiB per device) are made by the first large transfer of
-// any context on a device, shared by its contexts, and given back when the last context that used
-// them is destroyed.  One transfer uses them at a time; a transfer that finds them busy (or could
-// not make them) takes the plain copy.
+// The workers and their pinned chunks (32 MiB per device) are shared by the device's contexts and
+// given back when the last context that used them is destroyed.  Making and giving them back takes
+// 1.3 ms (2.5-4.5 ms more the first time in a process), which a context of one upload and one
+// download does not get back below some 20 MiB: created, uploaded, run for 2 steps, downloaded and
+// destroyed with workers of its own against the plain copies, 4 MiB 3.4 against 1.6 ms, 10 MiB
+// 5.0 / 4.3, 16 MiB 6.25 / 6.2, 24 MiB 8.5 / 9.0, 48 MiB 14 / 17, 164 MiB 58 / 71.  So a context
+// has them made when its own transfers amount to BUILD_BYTES (HostTransfers) and uses those that
+// another context has had made from its first transfer on.  One transfer uses them at a time; a
+// transfer that finds them busy (or could not make them) takes the plain copy.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <atomic>
@@ -29,9 +34,10 @@ class HostCopy {
   static constexpr size_t CHUNK = (size_t)4 << 20;
   // below this the plain copy (a transfer needs chunks for more than one worker)
   static constexpr size_t MIN_BYTES = (size_t)4 << 20;
+  static constexpr size_t BUILD_BYTES = (size_t)64 << 20;
 
-  // The device's workers (made if there are none); null if that fails.
-  static std::shared_ptr<HostCopy> get(int dev) noexcept
+  // The device's workers; where there are none, made if `make` says so (null if that fails), else null.
+  static std::shared_ptr<HostCopy> get(int dev, bool make) noexcept
   {
     constexpr int MAXDEV = 64;
     static std::mutex mu;
@@ -40,7 +46,7 @@ class HostCopy {
     try {
       std::lock_guard<std::mutex> lk(mu);
       std::shared_ptr<HostCopy> p = live[dev].lock();
-      if (!p) {
+      if (!p && make) {
         p.reset(new HostCopy(dev));
         if (!p->start()) return nullptr;
         live[dev] = p;
@@ -244,7 +250,10 @@ class HostTransfers {
   {
     const bool up = kind == hipMemcpyHostToDevice;
     if (bytes >= HostCopy::MIN_BYTES && pageable_host(up ? src : dst)) {
-      if (!workers_) workers_ = HostCopy::get(device);
+      if (!workers_) {
+        moved_ += bytes;
+        workers_ = HostCopy::get(device, moved_ >= HostCopy::BUILD_BYTES);
+      }
       hipError_t e = hipSuccess;
       if (workers_ && workers_->copy(dst, src, bytes, up, stream, &e)) return e;
     }
@@ -253,7 +262,8 @@ class HostTransfers {
   }
 
  private:
-  std::shared_ptr<HostCopy> workers_;  // from the first large transfer on
+  std::shared_ptr<HostCopy> workers_;
+  size_t moved_ = 0;  // bytes of the transfers so far that the workers could have taken
 };
 
 }  // namespace fx

@@ -46,12 +46,39 @@ int other_device()
   return 0;
 }
 
+// contexts of one upload and one download each have no workers made; those of a busier context
+// serve all of the device and go with the last that used them
+int workers_where_they_repay()
+{
+  fakeStream st{0};
+  for (int request = 0; request < 3; request++) {
+    HostTransfers t;
+    t.device = 0;
+    REQUIRE(round_trip(t, st, 20 * MIB));
+  }
+  REQUIRE(fake::mallocs == 0 && fake::staged == 0);
+  HostTransfers *a = new HostTransfers, *b = new HostTransfers;
+  a->device = b->device = 0;
+  for (int r = 0; r < 4; r++) REQUIRE(round_trip(*a, st, 20 * MIB));
+  REQUIRE(fake::pinned > 0 && fake::staged > 0);
+  const int chunks = fake::mallocs, staged = fake::staged;
+  REQUIRE(round_trip(*b, st, 20 * MIB));
+  REQUIRE(fake::mallocs == chunks && fake::staged > staged);
+  delete a;
+  REQUIRE(fake::pinned == chunks);
+  REQUIRE(round_trip(*b, st, 20 * MIB));
+  delete b;
+  REQUIRE(fake::pinned == 0);
+  return 0;
+}
+
 }  // namespace
 
 int main(int, char **argv)
 {
   const std::string check = argv[1];
   if (check == "other_device") return other_device();
+  if (check == "workers_where_they_repay") return workers_where_they_repay();
   std::printf("no check %s\n", argv[1]);
   return 2;
 }

@@ -26,6 +26,23 @@ def random_state(e, seed):
     return U
 
 
+def busy_context():
+    """A context whose transfers have had the device's copying threads made."""
+    e = context(40 * MIB // NODE_BYTES)
+    U = random_state(e, 5)
+    e.upload(U)
+    assert np.array_equal(e.download(), U)
+    return e
+
+
+@pytest.fixture
+def workers():
+    e = busy_context()
+    yield
+    e.close()
+
+
+@pytest.mark.usefixtures("workers")
 @pytest.mark.parametrize("nbytes", [64 << 10, 4 * MIB, 8 * MIB, 33 * MIB])
 @pytest.mark.parametrize("step", [0, 1])
 def test_state_round_trip(nbytes, step):
@@ -38,6 +55,7 @@ def test_state_round_trip(nbytes, step):
 
 
 def test_contexts_transfer_at_once():
+    first = busy_context()
     es = [context(6000 + 7 * i) for i in range(3)]
     bad = []
 
@@ -54,10 +72,6 @@ def test_contexts_transfer_at_once():
     for t in th:
         t.join()
     assert not bad
-    for e in es:
+    for e in [first] + es:
         e.close()
-    e = context(6000)  # the workers are made again after the last context gave them back
-    U = random_state(e, 99)
-    e.upload(U)
-    assert np.array_equal(e.download(), U)
-    e.close()
+    busy_context().close()  # the workers are made again after the last context gave them back
