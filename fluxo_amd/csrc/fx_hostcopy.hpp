@@ -4,7 +4,7 @@
 // Here a few worker threads each copy chunks between the caller's array and two pinned chunks of
 // their own while the copy engine moves the others; page faults of a new destination are taken by
 // all of them at once.  84 MB (32^3 elements, N = 3): to the device 2.85 -> 1.96 ms, back into a new
-// array 8.2 -> 2.7 ms; 164 MB 5.5 -> 3.7 and 15.6 -> 4.3 ms; 10.5 MB 0.32 -> 0.31 and 0.60 -> 0.40 ms.
+// array 8.2 -> 2.7 ms; 164 MB 5.5 -> 3.7 and 15.6 -> 4.3 ms; 10.5 MB back 0.60 -> 0.40 ms.
 // (Pinned copies run at 57 GB/s here.)  Chunks of 1 and 2 MiB: every copy costs about 35 us of
 // its own, 84 MB up in 2.75 and 2.15 ms; 8 MiB loses on small transfers; 8 workers gain nothing.
 //
@@ -32,8 +32,11 @@ class HostCopy {
  public:
   static constexpr int WORKERS = 4;
   static constexpr size_t CHUNK = (size_t)4 << 20;
-  // below this the plain copy (a transfer needs chunks for more than one worker)
-  static constexpr size_t MIN_BYTES = (size_t)4 << 20;
+  // below these the plain copy.  To the device it is as fast up to 12 MiB (staged / plain: 4 MiB
+  // 0.16-0.20 / 0.144 ms, 8 MiB 0.27-0.31 / 0.253, 12 MiB 0.36 / 0.36, 16 MiB 0.46 / 0.47, 24 MiB
+  // 0.65 / 0.69), from it while one worker has all of it (4 MiB 0.25 / 0.25, 5 MiB 0.25-0.28 / 0.305,
+  // 8 MiB 0.36 / 0.48).
+  static constexpr size_t MIN_UP = (size_t)16 << 20, MIN_DOWN = (size_t)5 << 20;
   static constexpr size_t BUILD_BYTES = (size_t)64 << 20;
 
   // The device's workers; where there are none, made if `make` says so (null if that fails), else null.
@@ -249,7 +252,7 @@ class HostTransfers {
   hipError_t copy(void *dst, const void *src, size_t bytes, hipMemcpyKind kind, hipStream_t stream) noexcept
   {
     const bool up = kind == hipMemcpyHostToDevice;
-    if (bytes >= HostCopy::MIN_BYTES && pageable_host(up ? src : dst)) {
+    if (bytes >= (up ? HostCopy::MIN_UP : HostCopy::MIN_DOWN) && pageable_host(up ? src : dst)) {
       if (!workers_) {
         moved_ += bytes;
         workers_ = HostCopy::get(device, moved_ >= HostCopy::BUILD_BYTES);

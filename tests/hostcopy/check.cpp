@@ -72,6 +72,24 @@ int workers_where_they_repay()
   return 0;
 }
 
+// the sizes at which the staged copy takes over, for each direction
+int sizes()
+{
+  fakeStream st{0};
+  HostTransfers t;
+  t.device = 0;
+  for (int r = 0; r < 2; r++) REQUIRE(round_trip(t, st, 40 * MIB));
+  std::vector<char> a(16 * MIB), b(16 * MIB);
+  auto staged = [&](hipMemcpyKind kind, size_t bytes) {
+    const int before = fake::staged, plain = fake::plain;
+    if (t.copy(b.data(), a.data(), bytes, kind, &st) != hipSuccess) return -1;
+    return (fake::staged > before) != (fake::plain > plain) ? (int)(fake::staged > before) : -1;
+  };
+  REQUIRE(staged(hipMemcpyHostToDevice, 16 * MIB - 1) == 0 && staged(hipMemcpyHostToDevice, 16 * MIB) == 1);
+  REQUIRE(staged(hipMemcpyDeviceToHost, 5 * MIB - 1) == 0 && staged(hipMemcpyDeviceToHost, 5 * MIB) == 1);
+  return 0;
+}
+
 }  // namespace
 
 int main(int, char **argv)
@@ -79,6 +97,7 @@ int main(int, char **argv)
   const std::string check = argv[1];
   if (check == "other_device") return other_device();
   if (check == "workers_where_they_repay") return workers_where_they_repay();
+  if (check == "sizes") return sizes();
   std::printf("no check %s\n", argv[1]);
   return 2;
 }
