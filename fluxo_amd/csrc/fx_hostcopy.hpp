@@ -255,7 +255,9 @@ class HostTransfers {
     if (bytes >= (up ? HostCopy::MIN_UP : HostCopy::MIN_DOWN) && pageable_host(up ? src : dst)) {
       if (!workers_) {
         moved_ += bytes;
-        workers_ = HostCopy::get(device, moved_ >= HostCopy::BUILD_BYTES);
+        const bool make = moved_ >= HostCopy::BUILD_BYTES && !refused_;
+        workers_ = HostCopy::get(device, make);
+        refused_ = refused_ || (make && !workers_);  // no memory or threads for them: not asked for again
       }
       hipError_t e = hipSuccess;
       if (workers_ && workers_->copy(dst, src, bytes, up, stream, &e)) return e;
@@ -266,6 +268,7 @@ class HostTransfers {
 
  private:
   std::shared_ptr<HostCopy> workers_;
+  bool refused_ = false;
   size_t moved_ = 0;  // bytes of the transfers so far that the workers could have taken
 };
 

@@ -90,6 +90,24 @@ int sizes()
   return 0;
 }
 
+// without memory for the chunks: plain copies, and one attempt a context
+int no_memory()
+{
+  fakeStream st{0};
+  fake::no_memory = true;
+  HostTransfers t;
+  t.device = 0;
+  for (int r = 0; r < 4; r++) REQUIRE(round_trip(t, st, 70 * MIB));
+  REQUIRE(fake::mallocs == 1 && fake::staged == 0 && fake::plain == 8);
+  fake::no_memory = false;
+  HostTransfers u;
+  u.device = 0;
+  REQUIRE(round_trip(u, st, 70 * MIB) && fake::staged > 0);
+  const int plain = fake::plain;
+  REQUIRE(round_trip(t, st, 70 * MIB) && fake::plain == plain);  // another context's workers
+  return 0;
+}
+
 }  // namespace
 
 int main(int, char **argv)
@@ -98,6 +116,7 @@ int main(int, char **argv)
   if (check == "other_device") return other_device();
   if (check == "workers_where_they_repay") return workers_where_they_repay();
   if (check == "sizes") return sizes();
+  if (check == "no_memory") return no_memory();
   std::printf("no check %s\n", argv[1]);
   return 2;
 }

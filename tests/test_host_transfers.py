@@ -18,7 +18,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["other_device", "workers_where_they_repay", "sizes"])
+@pytest.mark.parametrize("check", ["other_device", "workers_where_they_repay", "sizes", "no_memory"])
 def test_host_transfers(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
