@@ -704,7 +704,8 @@ int fx_tune_volume(fx_ctx *c, int reps, int *best_epb, int *tiles, double *ms, i
   (void)hipEventDestroy(e1);
   cleanup();
   b.vol_tile = best;
-  tuned_tile(N, b.cfg.parabolic, b.cfg.precision) = best;
+  // a context without alternatives leaves the choice of those that have them alone
+  if (ranocha) tuned_tile(N, b.cfg.parabolic, b.cfg.precision) = best;
   if (c->graph) { (void)hipGraphExecDestroy(c->graph); c->graph = nullptr; }
   if (best_epb) *best_epb = tile_epb(N, best);
   if (ntiles) *ntiles = nt;
