@@ -205,6 +205,12 @@ k_face_table(const int *__restrict__ e2s, const int *__restrict__ s2e, int e0, i
 // defaults: N = 5 (13^3 elements, Euler) 65 -> 39 us, N = 4 (15 x 14 x 13, Navier-Stokes) 54.9 ->
 // 29.2 us, N = 3 8.5 -> 7.1 us (8^3, Euler) and 161 -> 146 us (32^3, Navier-Stokes); at N = 2
 // (24^3, Navier-Stokes) the line form takes 26.3 us, the node form 28.6 us.
+// The other fluxes, line -> node, LSERK kernel: N = 5 (12^3) 1.69-1.94 times as fast, N = 4 (15^3)
+// 1.49-1.79, N = 3 1.13-1.24 (8^3), 1.06-1.13 (12^3), 0.93-1.18 (16^3), 0.91-1.07 (20^3), 0.93-1.10
+// (24^3), 1.01-1.09 (32^3), 1.00-1.10 (40^3); the least gain is flux 0's, Euler (16.4 -> 17.7 us at 16^3,
+// 29.2 -> 32.2 at 20^3, 45.9 -> 49.2 at 24^3, 121 -> 120 at 32^3).  As Ut alone 1.35-1.68 at N = 5, 4
+// and 1.12-1.22, 1.04-1.14, 0.92-1.15, 0.90-1.00, 0.95-1.11, 0.96-1.16, 0.98-1.19 at the sizes of N = 3.
+// The form goes by the degree alone: a request's result is the same bits on any mesh it shares.
 // The node form's default tile: one wavefront per block at N = 3 (its barriers cost nothing), the
 // fewest wavefronts that fill their lanes at N = 4 (2 elements in 250 of 256 threads; 1 and 3: 32 and
 // 37 us against 30), one element at N = 5 (2: 41 us against 39).
@@ -611,6 +617,11 @@ k_volume_node(double *__restrict__ U, const double *__restrict__ Mf, const doubl
   // 146 us) and N = 4 (30.1 -> 29.2 us at 15 x 14 x 13), for two more barriers; at N = 5 the LDS
   // does not bound the blocks per CU, and the barriers cost 2 us of 39.
   constexpr bool FACE1 = N <= 4;
+  // The pair loop is unrolled but for the fluxes that volume_flux gives at N = 3: unrolled, several of
+  // these kept more values alive than 4 waves per SIMD have registers for and spilled (LSERK kernel,
+  // Euler 32^3, line form / unrolled / not: flux 2 121 / 138 / 118 us, flux 8 122 / 138 / 119, flux 9
+  // 122 / 130 / 121; without spills, flux 3, 125 / 120 / 121).
+  constexpr int PAIRS = N == 3 && !two_point_halved(VF) ? 1 : N;
   constexpr int NFACE = MODE != VMODE_VOLINT ? EPB * NF * 5 : 0, NBUF = (NFV + 9) * NN;
   // node fields [NFV], metric vectors [9, component 3 d + c of direction d] (NN doubles each)
   __shared__ double s_buf[FACE1 ? (NBUF > NFACE ? NBUF : NFACE) : NBUF + NFACE];
@@ -703,7 +714,7 @@ k_volume_node(double *__restrict__ U, const double *__restrict__ Mf, const doubl
     const int pos = (d == 0) ? i : ((d == 1) ? j : k), stride = (d == 0) ? 1 : ((d == 1) ? n : n2);
     const double *sm = s_m + 3 * d * NN;
     const double mo[3] = {sm[tid], sm[NN + tid], sm[2 * NN + tid]};
-#pragma unroll
+#pragma unroll PAIRS
     for (int s = 1; s < n; s++) {
       const int t2 = tid + (pos + s < n ? s : s - n) * stride;
       double nb[NF_COUNT], mn[3], F[5];
