@@ -6,20 +6,17 @@
 
 namespace fx {
 
-template <int N, int VF, bool PARA, int MODE, int EPB>
+// VR: the arithmetic of the flux differencing, FP64 or FP32-split.
+template <int N, int VF, bool PARA, int MODE, typename VR, int EPB>
 void launch_volume_e(const Batch &b, RKArgs rk)
 {
   const int nb = (b.cfg.nElems + EPB - 1) / EPB;
   if (nb <= 0) return;
-  if constexpr (has_fp32(VF)) {
-    if (b.cfg.precision == FX_PREC_FP32_SPLIT) {
-      hipLaunchKernelGGL((k_volume<N, VF, PARA, MODE, float, EPB>), dim3(nb), dim3(VolGeom<N, EPB>::TB), 0, b.stream,
-                         b.U, b.Mf32, b.Mg32, b.Mh32, b.sJ, b.e2s, b.Flux, b.Uv, b.Ut, b.Uttmp, rk, b.cfg.nElems,
-                         b.cfg.kappa);
-      return;
-    }
-  }
-  if constexpr (volume_node_form(N))
+  if constexpr (sizeof(VR) == 4)
+    hipLaunchKernelGGL((k_volume<N, VF, PARA, MODE, float, EPB>), dim3(nb), dim3(VolGeom<N, EPB>::TB), 0, b.stream,
+                       b.U, b.Mf32, b.Mg32, b.Mh32, b.sJ, b.e2s, b.Flux, b.Uv, b.Ut, b.Uttmp, rk, b.cfg.nElems,
+                       b.cfg.kappa);
+  else if constexpr (volume_node_form(N))
     hipLaunchKernelGGL((k_volume_node<N, VF, PARA, MODE, EPB>), dim3(nb), dim3(NodeGeom<N, EPB>::T), 0, b.stream, b.U,
                        b.Mf, b.Mg, b.Mh, b.sJ, b.e2s, b.Flux, b.Uv, b.Ut, b.Uttmp, rk, b.cfg.nElems, b.cfg.kappa);
   else
@@ -28,37 +25,45 @@ void launch_volume_e(const Batch &b, RKArgs rk)
                        b.cfg.kappa);
 }
 
-// The LSERK form with the Ranocha flux has every tile of VolTiles<N>; other forms use their
+// The LSERK form with the Ranocha flux has the tiles of VolTiles<N>; other forms use their
 // precision's default tile.
-template <int N, int VF, bool PARA, int MODE>
+template <int N, int VF, bool PARA, int MODE, typename VR>
 void launch_volume_t(const Batch &b, RKArgs rk)
 {
   using V = VolTiles<N>;
   if constexpr (MODE == VMODE_RK && VF == 32) {
+    if constexpr (V::n == 4 && sizeof(VR) == 8)  // tile 3 is an FP64 one
+      if (b.vol_tile == 3) return launch_volume_e<N, VF, PARA, MODE, VR, V::T[3]>(b, rk);
     switch (b.vol_tile) {
-    case 1: launch_volume_e<N, VF, PARA, MODE, V::T[1]>(b, rk); break;
-    case 2: launch_volume_e<N, VF, PARA, MODE, V::T[2]>(b, rk); break;
-    case 3: launch_volume_e<N, VF, PARA, MODE, V::T[V::n - 1]>(b, rk); break;  // tile 3 exists where n = 4
-    default: launch_volume_e<N, VF, PARA, MODE, V::T[0]>(b, rk); break;
+    case 1: launch_volume_e<N, VF, PARA, MODE, VR, V::T[1]>(b, rk); break;
+    case 2: launch_volume_e<N, VF, PARA, MODE, VR, V::T[2]>(b, rk); break;
+    default: launch_volume_e<N, VF, PARA, MODE, VR, V::T[0]>(b, rk); break;
     }
-    return;
+  } else {
+    launch_volume_e<N, VF, PARA, MODE, VR, V::T[sizeof(VR) == 4 ? V::DEF32 : V::DEF64]>(b, rk);
   }
-  if (b.cfg.precision == FX_PREC_FP32_SPLIT) launch_volume_e<N, VF, PARA, MODE, V::T[V::DEF32]>(b, rk);
-  else launch_volume_e<N, VF, PARA, MODE, V::T[V::DEF64]>(b, rk);
+}
+
+template <int N, int VF, typename VR>
+void launch_volume_m(const Batch &b, int mode, RKArgs rk)
+{
+  const bool para = b.cfg.parabolic != 0;
+  if (mode == VMODE_VOLINT) launch_volume_t<N, VF, false, VMODE_VOLINT, VR>(b, rk);
+  else if (mode == VMODE_RK) {
+    if (para) launch_volume_t<N, VF, true, VMODE_RK, VR>(b, rk);
+    else launch_volume_t<N, VF, false, VMODE_RK, VR>(b, rk);
+  } else {
+    if (para) launch_volume_t<N, VF, true, VMODE_RHS, VR>(b, rk);
+    else launch_volume_t<N, VF, false, VMODE_RHS, VR>(b, rk);
+  }
 }
 
 template <int N, int VF>
 void launch_volume_v(const Batch &b, int mode, RKArgs rk)
 {
-  const bool para = b.cfg.parabolic != 0;
-  if (mode == VMODE_VOLINT) launch_volume_t<N, VF, false, VMODE_VOLINT>(b, rk);
-  else if (mode == VMODE_RK) {
-    if (para) launch_volume_t<N, VF, true, VMODE_RK>(b, rk);
-    else launch_volume_t<N, VF, false, VMODE_RK>(b, rk);
-  } else {
-    if (para) launch_volume_t<N, VF, true, VMODE_RHS>(b, rk);
-    else launch_volume_t<N, VF, false, VMODE_RHS>(b, rk);
-  }
+  if constexpr (has_fp32(VF))
+    if (b.cfg.precision == FX_PREC_FP32_SPLIT) return launch_volume_m<N, VF, float>(b, mode, rk);
+  launch_volume_m<N, VF, double>(b, mode, rk);
 }
 
 template <int N>

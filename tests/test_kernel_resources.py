@@ -1,4 +1,5 @@
 """What the built library's kernels take of the GPU, from the metadata the compiler writes into it."""
+import re
 import struct
 
 import msgpack
@@ -50,8 +51,34 @@ def instances(kernels, name):
     return {k: v for k, v in kernels.items() if k.startswith(f"_ZN2fx{len(name)}{name}I")}
 
 
-def test_node_form_at_n3_keeps_its_values_in_registers(kernels):
+def test_node_form_keeps_its_values_in_registers(kernels):
     """4 waves per SIMD leave 128 registers; a variant that spills loses more than the form gains."""
     spilled = {k: v[".private_segment_fixed_size"] for k, v in instances(kernels, "k_volume_node").items()
-               if "ILi3E" in k and v[".private_segment_fixed_size"]}
+               if v[".private_segment_fixed_size"]}
     assert not spilled
+
+
+TILES = {2: (7, 14, 3), 3: (4, 2, 8), 4: (5, 2, 3), 5: (3, 1, 2)}  # elements per block, those that the tuner may set
+
+
+def test_volume_kernels_are_those_a_launch_can_take(kernels):
+    """One tile per degree and precision, the default; the LSERK form with flux 32 all of the degree's
+    (a further one, 1, in FP64 at N = 3).  FP64 runs the node form from N = 3 on, FP32-split the line form."""
+    RK, seen = 1, set()
+    for name in list(instances(kernels, "k_volume")) + list(instances(kernels, "k_volume_node")):
+        m = re.match(r"_ZN2fx\d+k_volume(_node)?ILi(\d)ELi(\d+)ELb([01])ELi(\d)E([fd])?Li(\d+)EE", name)
+        node, (N, flux, para, mode), vr, epb = m[1], map(int, m.group(2, 3, 4, 5)), m[6], int(m[7])
+        fp32 = vr == "f"
+        assert bool(node) == (N >= 3 and not fp32), name
+        if fp32:
+            assert flux in (0, 5, 10, 32), name
+        prec = native.FX_PREC_FP32_SPLIT if fp32 else native.FX_PREC_FP64
+        default = native.volume_tile(N, False, prec)
+        if mode == RK and flux == 32:
+            assert epb in TILES[N] or (N == 3 and not fp32 and epb == 1), name
+        else:
+            assert epb == default, name
+        seen.add((N, flux, para, mode, fp32))
+    forms = [(0, 0), (1, 0), (0, 1), (1, 1), (0, 2)]  # (parabolic, mode)
+    assert seen == {(N, f, p, m, prec) for N in TILES for f in (*range(11), 32) for p, m in forms
+                    for prec in ((False, True) if f in (0, 5, 10, 32) else (False,))}
