@@ -660,11 +660,10 @@ k_mhd_dt_reduce(const double *__restrict__ dtElem, const double *__restrict__ dt
   __shared__ double s_dt[1024], s_c[1024];
   __shared__ int s_er[1024];
   const int tid = threadIdx.x;
-  double m = 1.79e308, mc = 1.79e308;
+  double m[2] = {1.79e308, 1.79e308};
   int er = 0;
-  dt_minimum<1024>(dtElem, errElem, tid, nElems, m, er);
-  dt_minimum<1024>(dtch1Elem, nullptr, tid, nElems, mc, er);
-  s_dt[tid] = m; s_c[tid] = mc; s_er[tid] = er;
+  dt_minimum<1024, 2>({dtElem, dtch1Elem}, errElem, 0, nElems, m, er);
+  s_dt[tid] = m[0]; s_c[tid] = m[1]; s_er[tid] = er;
   __syncthreads();
   for (int stp = 512; stp > 0; stp >>= 1) {
     if (tid < stp) {
