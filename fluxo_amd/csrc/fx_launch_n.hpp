@@ -275,20 +275,29 @@ void launch_dt_n(const Batch &b, double cfl, double dfl)
                      b.cfg.parabolic);
 }
 
+template <int N, int MODE, typename VR, bool PARA, int PARTS>
+void launch_mhd_volume_e(const Batch &b, const VR *Mf, const VR *Mg, const VR *Mh, RKArgs rk)
+{
+  using G = MhdVolGeom<N, PARTS>;
+  const int nb = (b.cfg.nElems + G::EPB - 1) / G::EPB;
+  if (nb <= 0) return;
+  hipLaunchKernelGGL((k_mhd_volume<N, MODE, VR, PARA, PARTS>), dim3(nb), dim3(G::T), 0, b.stream, b.U, Mf, Mg, Mh,
+                     b.sJ, b.e2s, b.Flux, b.FluxS, b.Uv, b.Ut, b.Uttmp, rk, b.cfg.nElems, b.mhd_args(), b.st);
+}
+
+template <int N, int MODE, typename VR, bool PARA>
+void launch_mhd_volume_s(const Batch &b, const VR *Mf, const VR *Mg, const VR *Mh, RKArgs rk)
+{
+  if constexpr (mhd_parts_elems(N) > 0)
+    if (b.cfg.nElems <= mhd_parts_elems(N)) return launch_mhd_volume_e<N, MODE, VR, PARA, 3>(b, Mf, Mg, Mh, rk);
+  launch_mhd_volume_e<N, MODE, VR, PARA, 1>(b, Mf, Mg, Mh, rk);
+}
+
 template <int N, int MODE, bool PARA>
 void launch_mhd_volume_p(const Batch &b, RKArgs rk)
 {
-  constexpr int EPB = MhdVolGeom<N>::EPB, T = MhdVolGeom<N>::T;
-  const int nb = (b.cfg.nElems + EPB - 1) / EPB;
-  if (nb <= 0) return;
-  if (b.cfg.precision == FX_PREC_FP32_SPLIT)
-    hipLaunchKernelGGL((k_mhd_volume<N, MODE, float, PARA>), dim3(nb), dim3(T), 0, b.stream, b.U, b.Mf32, b.Mg32,
-                       b.Mh32, b.sJ, b.e2s, b.Flux, b.FluxS, b.Uv, b.Ut, b.Uttmp, rk, b.cfg.nElems, b.mhd_args(),
-                       b.st);
-  else
-    hipLaunchKernelGGL((k_mhd_volume<N, MODE, double, PARA>), dim3(nb), dim3(T), 0, b.stream, b.U, b.Mf, b.Mg,
-                       b.Mh, b.sJ, b.e2s, b.Flux, b.FluxS, b.Uv, b.Ut, b.Uttmp, rk, b.cfg.nElems, b.mhd_args(),
-                       b.st);
+  if (b.cfg.precision == FX_PREC_FP32_SPLIT) launch_mhd_volume_s<N, MODE, float, PARA>(b, b.Mf32, b.Mg32, b.Mh32, rk);
+  else launch_mhd_volume_s<N, MODE, double, PARA>(b, b.Mf, b.Mg, b.Mh, rk);
 }
 
 template <int N, int MODE>

@@ -393,28 +393,38 @@ __device__ __forceinline__ void derigs_flux2(const R *L, const R *Rt, const R *h
 // Ut_tmp's and then U's, because interleaved with its loads they left L2 in parts (376 instead of
 // 250 MB written, 294 us), and U's old values come from LDS and the fields instead of memory.
 // Blocks of one element (7 at N = 2); N = 4 with two: 222 us.
+// PARTS = 3, one element a block: a node has a thread for each of its three directions, whose sums meet
+// in LDS.  A mesh whose blocks all run at once takes the time of one thread's chain of pairs, which
+// is a third: LSERK / right-hand side, FP64, one thread a node -> three, N = 2 9.9 -> 6.75 / 8.7 -> 5.6 us
+// (6^3 elements), 10.9 -> 9.1 / 9.1 -> 7.5 (10^3); N = 3 9.6 -> 7.3 / 8.9 -> 6.4 (6^3), 11.1 -> 9.3 /
+// 9.8 -> 8.1 (8^3); N = 4 11.3 -> 9.4 / 10.1 -> 8.4 (4^3), 12.3 -> 10.6 / 10.7 -> 9.0 (6^3); in FP32 as
+// much.  (With one pair a thread and its partner's half through LDS: 8.5 / 6.3, 10.9 / 7.8; 9.9 / 7.9,
+// 11.2 / 8.4; 10.4 / 8.1, 11.5 / 8.7.)  Beyond what 256 CUs hold at a time (in FP64 4, 2 and 1 blocks
+// each) it loses: N = 2 12^3 12.2 -> 14.7, N = 3 10^3 14.4 -> 16.9, N = 4 7^3 15.8 -> 18.7.  At N = 5 a
+// block of 11 wavefronts leaves no registers for it (resistive LSERK 12.7 -> 14.0 us at 2^3).
+constexpr int mhd_parts_elems(int N) { return N == 2 ? 1024 : (N == 3 ? 512 : (N == 4 ? 256 : 0)); }
 template <int N> struct MhdGeom;
 template <> struct MhdGeom<2> { static constexpr int EPB = 7; };
 template <> struct MhdGeom<3> { static constexpr int EPB = 1; };
 template <> struct MhdGeom<4> { static constexpr int EPB = 1; };
 template <> struct MhdGeom<5> { static constexpr int EPB = 1; };
-template <int N> struct MhdVolGeom {
-  static constexpr int n3 = (N + 1) * (N + 1) * (N + 1), EPB = MhdGeom<N>::EPB;
-  static constexpr int T = ((EPB * n3 + 63) / 64) * 64;
+template <int N, int PARTS> struct MhdVolGeom {
+  static constexpr int n3 = (N + 1) * (N + 1) * (N + 1), EPB = PARTS == 1 ? MhdGeom<N>::EPB : 1;
+  static constexpr int T = ((PARTS * EPB * n3 + 63) / 64) * 64;
 };
 // the node fields that derigs_flux2 reads, in LDS slots
 constexpr int MFS_COUNT = 12;
 __host__ __device__ constexpr int mfs_slot(int f) { return f <= MF_LNBETA ? f : MF_LNBETA + 1; }  // MF_BB last
 
-template <int N, int MODE, typename VR, bool PARA>
-__global__ void __launch_bounds__(MhdVolGeom<N>::T, sizeof(VR) == 4 ? 4 : 3)
+template <int N, int MODE, typename VR, bool PARA, int PARTS>
+__global__ void __launch_bounds__((MhdVolGeom<N, PARTS>::T), (PARTS > 1 ? 1 : (sizeof(VR) == 4 ? 4 : 3)))
 k_mhd_volume(double *__restrict__ U, const VR *__restrict__ Mf, const VR *__restrict__ Mg, const VR *__restrict__ Mh,
              const double *__restrict__ sJ, const int *__restrict__ e2s, const double *__restrict__ FluxM,
              const double *__restrict__ FluxS, const double *__restrict__ Uv, double *__restrict__ Ut,
              double *__restrict__ Uttmp, RKArgs rk, int nElems, MhdArgs a, const DtState *__restrict__ st)
 {
   constexpr int n = N + 1, n2 = n * n, n3 = n2 * n, NF = 6 * n2;
-  constexpr int EPB = MhdVolGeom<N>::EPB, T = MhdVolGeom<N>::T, NN = EPB * n3;
+  constexpr int EPB = MhdVolGeom<N, PARTS>::EPB, T = MhdVolGeom<N, PARTS>::T, NN = EPB * n3;
   // the face terms' memory becomes the node fields' and the metric vectors'
   constexpr size_t FACEB = MODE != VMODE_VOLINT ? (size_t)EPB * NF * MV * 8 : 0, BUFB = (size_t)(MFS_COUNT + 9) * NN * sizeof(VR);
   __shared__ __align__(16) unsigned char s_raw[FACEB > BUFB ? FACEB : BUFB];
@@ -425,8 +435,9 @@ k_mhd_volume(double *__restrict__ U, const VR *__restrict__ Mf, const VR *__rest
   double *s_face = reinterpret_cast<double *>(s_raw);
   const Ops &op = c_ops[N];
   const int tid = threadIdx.x, e0 = blockIdx.x * EPB;
-  const int el = tid / n3, node = tid - el * n3, e = e0 + el;
-  const int prob = (tid < NN && e < nElems) ? elem_problem(rk.eprob, e) : -1;
+  const int part = PARTS == 1 ? 0 : tid / NN, at = PARTS == 1 ? tid : tid - part * NN;
+  const int el = at / n3, node = at - el * n3, e = e0 + el;
+  const int prob = (at < NN && part < PARTS && e < nElems) ? elem_problem(rk.eprob, e) : -1;
   const bool active = prob >= 0;
   const size_t c = (size_t)e * n3 + node;
   const int i = node % n, j = (node / n) % n, k = node / n2;
@@ -435,15 +446,21 @@ k_mhd_volume(double *__restrict__ U, const VR *__restrict__ Mf, const VR *__rest
     s_ds[s1][p1] = VR(op.Dsh[p1][l1 < n ? l1 : l1 - n]);
   }
   double u[MV];
-  VR m[9];
+  VR m[9 / PARTS];
   if (active) {
 #pragma unroll
     for (int v = 0; v < MV; v++) u[v] = U[c * MV + v];
+    if constexpr (PARTS == 1) {
 #pragma unroll
-    for (int q = 0; q < 3; q++) {
-      m[q] = Mf[c * 3 + q];
-      m[3 + q] = Mg[c * 3 + q];
-      m[6 + q] = Mh[c * 3 + q];
+      for (int q = 0; q < 3; q++) {
+        m[q] = Mf[c * 3 + q];
+        m[3 + q] = Mg[c * 3 + q];
+        m[6 + q] = Mh[c * 3 + q];
+      }
+    } else {
+      const VR *M = part == 0 ? Mf : (part == 1 ? Mg : Mh);
+#pragma unroll
+      for (int q = 0; q < 3; q++) m[q] = M[c * 3 + q];
     }
   }
   double fs[MV];  // the node's surface terms
@@ -467,7 +484,7 @@ k_mhd_volume(double *__restrict__ U, const VR *__restrict__ Mf, const VR *__rest
       for (int v = 0; v < MV; v++) s_face[it * MV + v] = F[v] * sg;
     }
     __syncthreads();
-    if (active) {
+    if (active && part == 0) {
       const NodeFaces nf = node_faces<N>(i, j, k);
 #pragma unroll
       for (int t = 0; t < 3; t++) {
@@ -486,65 +503,85 @@ k_mhd_volume(double *__restrict__ U, const VR *__restrict__ Mf, const VR *__rest
 #pragma unroll
     for (int q = 0; q < MF_COUNT; q++) {
       own[q] = VR(f[q]);
-      if (q <= MF_LNBETA || q == MF_BB) s_f[mfs_slot(q) * NN + tid] = own[q];
+      if (part == 0 && (q <= MF_LNBETA || q == MF_BB)) s_f[mfs_slot(q) * NN + at] = own[q];
     }
 #pragma unroll
-    for (int q = 0; q < 9; q++) s_m[q * NN + tid] = VR(0.5) * m[q];
-    if (MODE == VMODE_RK) {
+    for (int q = 0; q < 9 / PARTS; q++) s_m[(part * 3 + q) * NN + at] = VR(0.5) * m[q];
+    if (MODE == VMODE_RK && part == 0) {
 #pragma unroll
-      for (int v = 1; v < 5; v++) s_u[(v - 1) * NN + tid] = u[v];
+      for (int v = 1; v < 5; v++) s_u[(v - 1) * NN + at] = u[v];
       if (sizeof(VR) == 4) {
 #pragma unroll
-        for (int v = 4; v < MV; v++) s_u[v * NN + tid] = u[v == 4 ? 0 : v];
+        for (int v = 4; v < MV; v++) s_u[v * NN + at] = u[v == 4 ? 0 : v];
       }
     }
   }
+  // the node pass's inputs: after the pairs where their registers would cost a wave per SIMD
+  double tt[MV], uv[7], sj = 0.0;
+  auto node_inputs = [&]() {
+    if (MODE == VMODE_RK) {
+#pragma unroll
+      for (int v = 0; v < MV; v++) tt[v] = rk.first ? 0.0 : Uttmp[c * MV + v];
+    }
+    if (MODE != VMODE_VOLINT) {
+      if (PARA) {
+#pragma unroll
+        for (int v = 0; v < 7; v++) uv[v] = Uv[c * 7 + v];
+      }
+      sj = sJ[c];
+    }
+  };
+  if (PARTS > 1 && active && part == 0) node_inputs();
   __syncthreads();
-  if (!active) return;
+  if (PARTS == 1 && !active) return;
   const VR ch = VR(st->glm_ch), smu0 = VR(a.smu0), skm1 = VR(1.0 / (a.kappa - 1.0));
   VR acc[MV], pw = VR(0);
 #pragma unroll
   for (int v = 0; v < MV; v++) acc[v] = VR(0);
   constexpr int PAIR_UNROLL = sizeof(VR) == 8 ? 2 : 1;  // FP64 by 1 spills, by 4 as fast; FP32 by 2: +2 %
+  if (PARTS == 1 || active) {
 #pragma unroll 1
-  for (int d = 0; d < 3; d++) {
-    const int pos = (d == 0) ? i : ((d == 1) ? j : k), stride = (d == 0) ? 1 : ((d == 1) ? n : n2);
-    const VR *sm = s_m + 3 * d * NN;
-    const VR mo[3] = {sm[tid], sm[NN + tid], sm[2 * NN + tid]};
+    for (int d = part; d < (PARTS == 1 ? 3 : part + 1); d++) {
+      const int pos = (d == 0) ? i : ((d == 1) ? j : k), stride = (d == 0) ? 1 : ((d == 1) ? n : n2);
+      const VR *sm = s_m + 3 * d * NN;
+      const VR mo[3] = {sm[at], sm[NN + at], sm[2 * NN + at]};
 #pragma unroll PAIR_UNROLL
-    for (int s = 1; s < n; s++) {
-      const int t2 = tid + (pos + s < n ? s : s - n) * stride;
-      VR nb[MF_COUNT], mn[3], F[MV], Bm;
+      for (int s = 1; s < n; s++) {
+        const int t2 = at + (pos + s < n ? s : s - n) * stride;
+        VR nb[MF_COUNT], mn[3], F[MV], Bm;
 #pragma unroll
-      for (int q = 0; q < MF_COUNT; q++)
-        nb[q] = (q <= MF_LNBETA || q == MF_BB) ? s_f[mfs_slot(q) * NN + t2] : VR(0);
+        for (int q = 0; q < MF_COUNT; q++)
+          nb[q] = (q <= MF_LNBETA || q == MF_BB) ? s_f[mfs_slot(q) * NN + t2] : VR(0);
 #pragma unroll
-      for (int q = 0; q < 3; q++) mn[q] = sm[q * NN + t2];
-      derigs_flux2<VR>(own, nb, mo, mn, ch, smu0, skm1, F, Bm);
-      const VR ds = s_ds[s - 1][pos];
+        for (int q = 0; q < 3; q++) mn[q] = sm[q * NN + t2];
+        derigs_flux2<VR>(own, nb, mo, mn, ch, smu0, skm1, F, Bm);
+        const VR ds = s_ds[s - 1][pos];
 #pragma unroll
-      for (int v = 0; v < MV; v++) acc[v] += ds * F[v];
-      pw += ds * Bm;
+        for (int v = 0; v < MV; v++) acc[v] += ds * F[v];
+        pw += ds * Bm;
+      }
+      // the pair of the node with itself: its Dvolsurf row sum is what the others leave
+      pw += VR(op.DsRow[pos]) * (mo[0] * own[MF_B1] + mo[1] * own[MF_B2] + mo[2] * own[MF_B3]);
     }
-    // the pair of the node with itself: its Dvolsurf row sum is what the others leave
-    pw += VR(op.DsRow[pos]) * (mo[0] * own[MF_B1] + mo[1] * own[MF_B2] + mo[2] * own[MF_B3]);
+    acc[1] += pw * own[MF_B1]; acc[2] += pw * own[MF_B2]; acc[3] += pw * own[MF_B3];
+    acc[4] += pw * own[MF_VB];
+    acc[5] += pw * own[MF_V1]; acc[6] += pw * own[MF_V2]; acc[7] += pw * own[MF_V3];
   }
-  acc[1] += pw * own[MF_B1]; acc[2] += pw * own[MF_B2]; acc[3] += pw * own[MF_B3];
-  acc[4] += pw * own[MF_VB];
-  acc[5] += pw * own[MF_V1]; acc[6] += pw * own[MF_V2]; acc[7] += pw * own[MF_V3];
-  // the node pass: its loads first, its stores last and contiguous
-  double tt[MV], uv[7], sj = 0.0;
-  if (MODE == VMODE_RK) {
+  if constexpr (PARTS > 1) {  // the directions' sums meet where the fields were
+    VR *s_x = s_f;
+    __syncthreads();
+    if (active && part > 0) {
 #pragma unroll
-    for (int v = 0; v < MV; v++) tt[v] = rk.first ? 0.0 : Uttmp[c * MV + v];
-  }
-  if (MODE != VMODE_VOLINT) {
-    if (PARA) {
-#pragma unroll
-      for (int v = 0; v < 7; v++) uv[v] = Uv[c * 7 + v];
+      for (int v = 0; v < MV; v++) s_x[((part - 1) * MV + v) * NN + at] = acc[v];
     }
-    sj = sJ[c];
+    __syncthreads();
+    if (!active || part > 0) return;
+#pragma unroll
+    for (int v = 0; v < MV; v++) acc[v] = acc[v] + s_x[v * NN + at] + s_x[(MV + v) * NN + at];
+  } else {
+    node_inputs();
   }
+  // the node pass: its stores last and contiguous
   double tot[MV];
 #pragma unroll
   for (int v = 0; v < MV; v++) tot[v] = double(acc[v]);
@@ -559,12 +596,12 @@ k_mhd_volume(double *__restrict__ U, const VR *__restrict__ Mf, const VR *__rest
   if (MODE == VMODE_RK) {
     const double bdt = rk.b * rk.st[prob].dt;
 #pragma unroll
-    for (int v = 1; v < 5; v++) u[v] = s_u[(v - 1) * NN + tid];
+    for (int v = 1; v < 5; v++) u[v] = s_u[(v - 1) * NN + at];
     if (sizeof(VR) == 8) {  // the fields rho, B and psi are the state's own values
       u[0] = own[MF_RHO]; u[5] = own[MF_B1]; u[6] = own[MF_B2]; u[7] = own[MF_B3]; u[8] = own[MF_PSI];
     } else {
 #pragma unroll
-      for (int v = 4; v < MV; v++) u[v == 4 ? 0 : v] = s_u[v * NN + tid];
+      for (int v = 4; v < MV; v++) u[v == 4 ? 0 : v] = s_u[v * NN + at];
     }
 #pragma unroll
     for (int v = 0; v < MV; v++) tt[v] = rk.first ? tot[v] : tt[v] * (-rk.A) + tot[v];

@@ -39,8 +39,12 @@ def test_node_form_against_oracle(N, K, flux, nfvse):
     e.close()
 
 
-@pytest.mark.parametrize("N", [2, 3, 4, 5])
-@pytest.mark.parametrize("K", [(1, 1, 1), (2, 2, 2), (3, 5, 1)])
+# at each degree up to its largest mesh of three threads a node, and the first ones with one
+MHD_MESHES = [(N, K) for N in (2, 3, 4, 5) for K in ((1, 1, 1), (2, 2, 2), (3, 5, 1))] + [
+    (2, (16, 8, 8)), (2, (41, 5, 5)), (3, (8, 8, 8)), (3, (19, 9, 3)), (4, (8, 8, 4)), (4, (13, 5, 4))]
+
+
+@pytest.mark.parametrize("N,K", MHD_MESHES)
 @pytest.mark.parametrize("resistive", [False, True])
 def test_mhd_node_form_against_oracle(N, K, resistive):
     """The GLM-MHD volume kernel in FP64 (bar 1e-12) and FP32-split (2e-5: FP32 rounding of
