@@ -257,18 +257,20 @@ enum { FX_KERNEL_VOLUME_RK = 0, FX_KERNEL_SURFACE = 1, FX_KERNEL_LIFTING = 2, FX
        FX_KERNEL_VOLUME_RHS = 4, FX_KERNEL_NFVSE_ALPHA = 5, FX_KERNEL_NFVSE_FV = 6 };
 int fx_profile_kernel(fx_ctx *ctx, int which, int reps, double *avg_ms);
 
-/* Tile tuner of the volume kernel (no counterpart in the reference).  Times each compiled
-   tile (elements per workgroup) of the LSERK volume kernel on this context's mesh and
-   state, restores U and Ut_tmp, and keeps the fastest for this context and as the
-   process-wide choice for its (N, parabolic, precision), used by contexts and server pools
-   created afterwards.
+/* Tile tuner of the volume kernel (no counterpart in the reference).  Times three tiles
+   (elements per workgroup: the default and two others) of the LSERK volume kernel on this
+   context's mesh and state, restores U and Ut_tmp, and keeps the fastest for this context
+   and as the process-wide choice for its (N, parabolic, precision), used by contexts and
+   server pools created afterwards.
    tiles[t] / ms[t] (room for 4) receive each candidate's elements per workgroup and average
    launch time, *ntiles their number, *best_epb the choice.  Only the Ranocha (VolumeFlux
-   32) form has alternatives; other fluxes report their single tile. */
+   32) form has alternatives; other fluxes and GLM-MHD report their single tile and leave
+   the process-wide choice as it is. */
 int fx_tune_volume(fx_ctx *ctx, int reps, int *best_epb, int *tiles, double *ms, int *ntiles);
 /* The process-wide volume-kernel tile (elements per workgroup) for (N, parabolic, precision). */
 int fx_volume_tile(int N, int parabolic, int precision, int *epb);
-/* Use the tile with epb elements per workgroup for this context (FX_EINVAL if none). */
+/* Use the tile with epb elements per workgroup for this context (FX_EINVAL if none): one of
+   those the tuner times, or 8 at N = 3 in FP64. */
 int fx_use_volume_tile(fx_ctx *ctx, int epb);
 
 /* Device bytes held by a context with this configuration (for HBM admission). */

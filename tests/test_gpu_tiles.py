@@ -3,7 +3,7 @@ import numpy as np
 import pytest
 
 from fluxo_amd.mesh import box_mesh
-from fluxo_amd.native import FX_PREC_FP32_SPLIT, FX_PREC_FP64, Engine, MhdEngine, volume_tile
+from fluxo_amd.native import FX_PREC_FP32_SPLIT, FX_PREC_FP64, Engine, FxError, MhdEngine, volume_tile
 from fluxo_amd.workloads import perturbed_orszag_tang, taylor_green
 
 pytestmark = pytest.mark.gpu
@@ -41,3 +41,32 @@ def test_tuning_without_alternatives_keeps_the_choice():
         _, times = tune(lambda: MhdEngine(m, resistive=res, precision=prec), perturbed_orszag_tang(m["Elem_xGP"], 3))
         assert len(times) == 1
     assert {k: volume_tile(*k) for k in keys} == tuned
+
+
+ACCEPTED = {(2, FX_PREC_FP64): {7, 14, 3}, (3, FX_PREC_FP64): {1, 4, 2, 8}, (4, FX_PREC_FP64): {5, 2, 3},
+            (5, FX_PREC_FP64): {3, 1, 2}, (2, FX_PREC_FP32_SPLIT): {7, 14, 3}, (3, FX_PREC_FP32_SPLIT): {4, 2, 8},
+            (4, FX_PREC_FP32_SPLIT): {5, 2, 3}, (5, FX_PREC_FP32_SPLIT): {3, 1, 2}}
+
+
+@pytest.mark.parametrize("N,precision", list(ACCEPTED))
+@pytest.mark.parametrize("parabolic", [False, True])
+def test_every_accepted_tile_gives_the_same_steps(N, precision, parabolic):
+    """Also a tile that the tuner does not time (8 at N = 3 in FP64); 27 elements leave the last block
+    partly filled, or are fewer than two blocks."""
+    m = box_mesh(3, N, Ngeo=3, warp=True, **TGV)
+    U = taylor_green(m["Elem_xGP"])
+    e = Engine(m, volume_flux=32, parabolic=parabolic, mu0=1.0 / 1600, precision=precision)
+    results = {}
+    for epb in range(17):
+        try:
+            e.use_volume_tile(epb)
+        except FxError:
+            continue
+        e.upload(U)
+        t, dt, err = e.run(3, 0.5, 0.5)
+        assert err == 0
+        results[epb] = e.download()
+    e.close()
+    assert set(results) == ACCEPTED[N, precision]
+    first = next(iter(results.values()))
+    assert all(np.array_equal(V, first) for V in results.values())
