@@ -1161,11 +1161,13 @@ k_lifting(const double *__restrict__ U, const double *__restrict__ Mf, const dou
   const int i = node % n, j = (node / n) % n, k = node / n2;
   const size_t c = (size_t)e * n3 + node;
   static_assert(!DT || (NV == 5 && OUT == 1), "CALCTIMESTEP in the Navier-Stokes stage lifting only");
-  // D and D_hat by column in LDS for the BR1 contractions without the matrix core: each lane reads
-  // its row's entry, which from constant memory is a vector load of its own (GLM-MHD N = 4, 24^3:
-  // 193 -> 178 us, Navier-Stokes N = 5: 44.6 -> 43 us; BR2 at N = 2 lost 1 us of 34 and keeps the
-  // constant memory)
-  constexpr bool LDSOP = N != 3 && LIFT == 1;
+  // D and D_hat by column in LDS for the contractions without the matrix core: each lane reads its
+  // row's entry, which from constant memory is a vector load of its own (BR1: GLM-MHD N = 4, 24^3
+  // 193 -> 178 us, Navier-Stokes N = 5 44.6 -> 43 us; BR2 with GLM-MHD: N = 2 24^3 79.8 -> 58.2, N = 3
+  // 24^3 187 -> 129, N = 4 15^3 91.7 -> 65.1, N = 5 12^3 88.6 -> 60.8, and 12.5 -> 13.0 to 15.0 -> 15.4 at
+  // 8^3).  BR2 with Navier-Stokes gains nothing, N = 2 24^3 36.1 -> 36.6, N = 3 75.8 -> 75.3, N = 4 15^3
+  // 41.3 -> 40.8, N = 5 12^3 37.1 -> 36.9, and loses 0.2 of 10.6 us at 8^3: it keeps the constant memory.
+  constexpr bool LDSOP = LIFT == 1 ? N != 3 : NV == 9;
   __shared__ double s_op[LDSOP ? 2 * n2 : 1];
   if (LDSOP && tid < n2) {
     s_op[tid] = op.D[tid % n][tid / n];
