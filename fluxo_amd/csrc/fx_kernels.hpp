@@ -595,8 +595,9 @@ k_volume(double *__restrict__ U, const VR *__restrict__ Mf, const VR *__restrict
 // direction sums and three to five of its six barriers.  The kernel holds 118-128 VGPR (4 waves per
 // SIMD) and is bound by its vector instructions at N = 4, 5 and by memory at N = 3 (633 MB in
 // 142-150 us at 32^3 elements, Navier-Stokes: 4.2-4.4 TB/s against 5.1 TB/s of a 1 GiB copy).
-// NodeGeom: EPB elements per block, T threads.  The lines of a direction are rotations of the node
-// index, so unpadded LDS arrays read without bank conflicts.
+// NodeGeom: EPB elements per block, T threads.  The LDS arrays are not padded: at N = 3 the partners
+// of 32 lanes are whole lines rotated, 32 different nodes and so every bank once; at N = 4 and 5 the
+// lanes of a wavefront straddle lines and some reads meet in a bank.
 template <int N, int EPB_> struct NodeGeom {
   static constexpr int n3 = (N + 1) * (N + 1) * (N + 1), EPB = EPB_;
   static constexpr int T = ((EPB * n3 + 63) / 64) * 64;

@@ -44,7 +44,7 @@ k_nfvse_alpha(const double *__restrict__ U, const int *__restrict__ eprob, doubl
   const bool active = el < EPB && e < nElems && elem_problem(eprob, e) >= 0;
   const int i = node % n, j = (node / n) % n, k = node / (n * n);
   // the modal operator by column: each lane reads its row's entries, which from constant memory are
-  // vector loads of their own (40^3 elements, N = 3: 47 -> 39 us; reading U at the rate of a large
+  // vector loads of their own (40^3 elements, N = 3: 49 -> 44 us; reading U at the rate of a large
   // copy takes 32 us)
   __shared__ double s_v[n * n];
   if (a.computeAlpha == 1) {

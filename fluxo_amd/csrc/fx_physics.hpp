@@ -732,7 +732,6 @@ __device__ __forceinline__ double face_lambda(const double *UL, const double *UR
   return fmax(fabs(mL / UL[0]), fabs(mR / UR[0])) + sqrt(fmax(c2L, c2R));
 }
 
-// ConsToEntropy (navierstokes/equation_vars.f90:362-391); s = -ln(rho_sp*rho^(kappa-1))
 // 1/rho, velocity, |v|^2/2 and pressure of a state.  The lifting kernel forms entropy variables,
 // primitive gradients and viscous fluxes from one state: as the same expressions they are evaluated
 // once per state, with one division each for 1/rho and rho/p.
@@ -747,7 +746,8 @@ struct PrimState {
   }
 };
 
-// is evaluated as -(ln rho_sp + (kappa-1) ln rho).
+// ConsToEntropy (navierstokes/equation_vars.f90:362-391); s = -ln(rho_sp*rho^(kappa-1)) is
+// evaluated as -(ln rho_sp + (kappa-1) ln rho).
 __device__ __forceinline__ void cons_to_entropy(const double *U, double kappa, double skappaM1, double *w)
 {
   const PrimState q(U, kappa);
