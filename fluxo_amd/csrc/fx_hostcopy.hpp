@@ -32,11 +32,12 @@ class HostCopy {
  public:
   static constexpr int WORKERS = 4;
   static constexpr size_t CHUNK = (size_t)4 << 20;
-  // below these the plain copy.  To the device it is as fast up to 12 MiB (staged / plain: 4 MiB
-  // 0.16-0.20 / 0.144 ms, 8 MiB 0.27-0.31 / 0.253, 12 MiB 0.36 / 0.36, 16 MiB 0.46 / 0.47, 24 MiB
-  // 0.65 / 0.69), from it while one worker has all of it (4 MiB 0.25 / 0.25, 5 MiB 0.25-0.28 / 0.305,
-  // 8 MiB 0.36 / 0.48).
-  static constexpr size_t MIN_UP = (size_t)16 << 20, MIN_DOWN = (size_t)5 << 20;
+  // below these the plain copy: to the device while the chunks occupy two workers at most (arrays
+  // not in the host's caches, plain / staged: 4 MiB 0.18 / 0.25 ms, 8 MiB 0.33 / 0.36, 10 MiB 0.40 / 0.36,
+  // 14 MiB 0.54 / 0.465, 20 MiB 0.77 / 0.65; one array sent again and again is as fast either way from 10
+  // to 16 MiB), from it while one worker has all of it (4 MiB 0.25 / 0.25, 5 MiB 0.30 / 0.255, 8 MiB
+  // 0.48 / 0.35).
+  static constexpr size_t MIN_UP = (size_t)9 << 20, MIN_DOWN = (size_t)5 << 20;
   static constexpr size_t BUILD_BYTES = (size_t)64 << 20;
 
   // The device's workers; where there are none, made if `make` says so (null if that fails), else null.

@@ -85,7 +85,7 @@ int sizes()
     if (t.copy(b.data(), a.data(), bytes, kind, &st) != hipSuccess) return -1;
     return (fake::staged > before) != (fake::plain > plain) ? (int)(fake::staged > before) : -1;
   };
-  REQUIRE(staged(hipMemcpyHostToDevice, 16 * MIB - 1) == 0 && staged(hipMemcpyHostToDevice, 16 * MIB) == 1);
+  REQUIRE(staged(hipMemcpyHostToDevice, 9 * MIB - 1) == 0 && staged(hipMemcpyHostToDevice, 9 * MIB) == 1);
   REQUIRE(staged(hipMemcpyDeviceToHost, 5 * MIB - 1) == 0 && staged(hipMemcpyDeviceToHost, 5 * MIB) == 1);
   return 0;
 }

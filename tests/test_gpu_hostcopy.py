@@ -43,7 +43,7 @@ def workers():
 
 
 @pytest.mark.usefixtures("workers")
-@pytest.mark.parametrize("nbytes", [64 << 10, 4 * MIB, 5 * MIB, 8 * MIB, 16 * MIB, 33 * MIB])
+@pytest.mark.parametrize("nbytes", [64 << 10, 4 * MIB, 5 * MIB, 8 * MIB, 9 * MIB, 33 * MIB])
 @pytest.mark.parametrize("step", [0, 1])
 def test_state_round_trip(nbytes, step):
     e = context(nbytes // NODE_BYTES + step)  # the last size below and the first above
