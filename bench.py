@@ -77,13 +77,13 @@ def volume_kernel_bytes(N, nElems, parabolic, metric_bytes=8):
 
 def lifting_kernel_bytes(N, nElems):
     """Algorithmic HBM bytes of one launch of the Navier-Stokes lifting kernel (viscous
-    form): U, metrics and sJ of every node; at each of the element's 6 faces the
-    neighbour's face-node state (5) and the face normal with SurfElem (4), located through the
-    face-point table (two 4-byte integers per face point); written: the 4-component viscous
-    volume term per node and the 4-component normal viscous flux at each of the 6 faces."""
+    form), each array read or written once: U, metrics and sJ of every node (the neighbours'
+    face-node states among them), the normal with SurfElem (4) of the element's 3 owned sides,
+    the face-point table (two 4-byte integers per element face point); written: the 4-component
+    viscous volume term per node and the 4-component normal viscous flux at each of the 6 faces."""
     n = N + 1
     n3, n2 = n ** 3, n ** 2
-    return (8 * (5 * n3 + 9 * n3 + n3 + 6 * n2 * 5 + 6 * n2 * 4 + 4 * n3 + 6 * n2 * 4) + 8 * 6 * n2) * nElems
+    return (8 * (5 * n3 + 9 * n3 + n3 + 3 * n2 * 4 + 4 * n3 + 6 * n2 * 4) + 8 * 6 * n2) * nElems
 
 
 def surface_kernel_bytes(N, nSides, parabolic):
