@@ -58,6 +58,7 @@ def test_node_form_keeps_its_values_in_registers(kernels):
     assert not spilled
 
 
+DEFAULT = {False: {2: 7, 3: 1, 4: 2, 5: 1}, True: {2: 7, 3: 4, 4: 5, 5: 3}}  # by FP32-split
 TILES = {2: (7, 14, 3), 3: (4, 2, 8), 4: (5, 2, 3), 5: (3, 1, 2)}  # elements per block, those that the tuner may set
 
 
@@ -72,12 +73,10 @@ def test_volume_kernels_are_those_a_launch_can_take(kernels):
         assert bool(node) == (N >= 3 and not fp32), name
         if fp32:
             assert flux in (0, 5, 10, 32), name
-        prec = native.FX_PREC_FP32_SPLIT if fp32 else native.FX_PREC_FP64
-        default = native.volume_tile(N, False, prec)
         if mode == RK and flux == 32:
             assert epb in TILES[N] or (N == 3 and not fp32 and epb == 1), name
         else:
-            assert epb == default, name
+            assert epb == DEFAULT[fp32][N], name
         seen.add((N, flux, para, mode, fp32))
     forms = [(0, 0), (1, 0), (0, 1), (1, 1), (0, 2)]  # (parabolic, mode)
     assert seen == {(N, f, p, m, prec) for N in TILES for f in (*range(11), 32) for p, m in forms
