@@ -1730,13 +1730,13 @@ k_calc_dt(const double *__restrict__ U, const double *__restrict__ Mf, const dou
 
 #ifdef FX_KERNEL_HOME  // non-template kernels: compiled in one unit only
 // Minima of ND arrays and the maximum error code over a block's entries i0 <= i < i1 (NaN entries
-// skipped: a comparison with NaN is false), T threads.  DTR entries a thread are loaded ahead of the
-// first comparison, then what is left in pieces of 4, 2 and 1; past the end the last entry again,
-// which changes no minimum.  At one load's latency per entry the one-block reduction of 64,000
-// elements took 24 us, now 17 us.  GLM-MHD's two arrays go in the same pass: one after the other, and
-// with what is left below DTR entries one by one, its CALCTIMESTEP (k_mhd_calc_dt and the reduction,
-// N = 3) took 10.3 us at 12^3 elements, 24.5 at 20^3 and 33.3 at 24^3, now 9.65, 21.9 and 31.2 (9.6,
-// 21.9 and 31.7 with one load at a time; at 64 and 512 elements 0.3 us of 8 more than that).
+// skipped: a comparison with NaN is false), T threads.  What does not fill DTR entries a thread goes
+// first, in pieces of 1, 2 and 4, the entries of a piece all loaded before its first comparison; past
+// the end the last entry again, which changes no minimum.  At one load's latency per entry the
+// one-block reduction of 64,000 elements took 24 us, now 16 us.  GLM-MHD's two arrays go in the same
+// pass: one after the other, and with the pieces one by one, its CALCTIMESTEP (k_mhd_calc_dt and the
+// reduction, N = 3) took 10.3 us at 12^3 elements, 24.4 at 20^3 and 33.4 at 24^3, now 9.6, 21.4 and 31.5
+// (9.6, 21.8 and 31.5 with one load at a time; at 64 and 512 elements 0.2 us of 8 more than that).
 constexpr int DTR = 8;
 template <int T, int ND, int Q>
 __device__ __forceinline__ void dt_entries(const double *const (&dt)[ND], const int *__restrict__ err, int i, int i1,
@@ -1764,10 +1764,12 @@ __device__ __forceinline__ void dt_minimum(const double *const (&dt)[ND], const 
                                            double (&m)[ND], int &er)
 {
   int i = i0 + threadIdx.x, left = (i1 - i0 + T - 1) / T;
-  for (; left >= DTR; left -= DTR, i += DTR * T) dt_entries<T, ND, DTR>(dt, err, i, i1, m, er);
-  if (left & 4) { dt_entries<T, ND, 4>(dt, err, i, i1, m, er); i += 4 * T; }
-  if (left & 2) { dt_entries<T, ND, 2>(dt, err, i, i1, m, er); i += 2 * T; }
-  if (left & 1) dt_entries<T, ND, 1>(dt, err, i, i1, m, er);
+  if (left & 1) { dt_entries<T, ND, 1>(dt, err, i, i1, m, er); i += T; }
+  if (__builtin_expect(left > 1, 0)) {  // out of the way of the small meshes' instruction fetches
+    if (left & 2) { dt_entries<T, ND, 2>(dt, err, i, i1, m, er); i += 2 * T; }
+    if (left & 4) { dt_entries<T, ND, 4>(dt, err, i, i1, m, er); i += 4 * T; }
+    for (left /= DTR; left > 0; left--, i += DTR * T) dt_entries<T, ND, DTR>(dt, err, i, i1, m, er);
+  }
 }
 
 // Minimum of dtElem (NaN entries skipped) and maximum error code, one block, fixed order.
